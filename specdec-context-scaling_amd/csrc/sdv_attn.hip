@@ -85,18 +85,14 @@ struct AttnArgs {
   // replays reuse it) and the bound of every cross-workgroup wait, in polls
   uint32_t tag;
   uint32_t spin_limit;
-  // prefill pass 2: key parts per row group (1: each workgroup writes its rows' outputs itself)
-  int pf_parts;
-  // prefill pass 1: key parts per row group (the (max, sum) of each, per row, in stats)
-  int pf_split;
-  // prefill pass 2 with parts per row group by its key count (pf_kstar > 0, S a multiple of
-  // the pass's rows per workgroup): at most pf_kstar blocks per part, pf_wh workgroups per
-  // head; pf_parts is then the most parts of any row group (its slots per row group)
-  int pf_kstar, pf_wh;
+  // prefill: row groups of the (layer, sequence, KV head) group; workgroups that share pass 1's
+  // and pass 2's stages evenly (0: a row group per workgroup) and the fewest stages of one;
+  // (max, sum) pairs per row (pass 1's segments); part slots in `partial` (the rest follow in
+  // the sync area's partials), and how they are numbered
+  int pf_nrg, pf_w1, pf_w2, pf_min1, pf_min2, pf_split, pf_slots, pf_dense;
   // prefill: V dequantized once per call by pass 1 for pass 2.  Per (layer, sequence, KV head)
-  // group, vh_stages stages of two page blocks, each D/16 dimension tiles x 64 lanes x 16 bytes
-  // in the lane order of the p.V MFMA's A operand (lane (g, n): dimension dt*16 + n, tokens
-  // 4g..4g+3 of the first block, then of the second)
+  // group, vh_stages pairs of page blocks, each block D/32 dimension tiles x 64 lanes x 16 bytes
+  // in the lane order of the p.V MFMA's A operand
   uint4* vhat;
   int vh_stages;
 };
@@ -1752,533 +1748,9 @@ __global__ void zero_kernel(uint32_t* p, size_t n) {
 }
 
 // ---------------------------------------------------------------------------- prefill
-// Shapes with more query rows than one row-tile group holds (R = G*S > 64: prefill and
-// chunked-prefill blocks, model_self.py:471-504, 637-648) in two launches whose workspace holds
-// the per-row (max, sum) of each key part -- 8 bytes per row and part -- and V dequantized once
-// (2 bytes per key and dimension of each KV head) instead of the O(S*T) scores:
-//   pass 1  each wavefront takes 32 rows (two MFMA row tiles) and streams one part of the page
-//           blocks its rows can see (one workgroup per part): S^T = K Q^T on MFMA (the K page is
-//           the A operand, the rows the B operand; one K operand serves both tiles), scores
-//           rounded to BF16 twice, offset-causal mask, online (max, sum) per lane, merged over
-//           the lane groups into the part's (max, sum) per row.  The launch also dequantizes
-//           V, each stage of two blocks once, as bf16(fp32(code) * scale) in the lane order of
-//           pass 2's MFMA operand.
-//   pass 2  merges the parts in part order into (M, L); each wavefront (32 rows) streams its
-//           part of the blocks again, recomputes its rows' BF16 scores and forms
-//           p = bf16(exp(s - M) / L) in registers.  A lane's S^T fragment (row n, tokens
-//           4g..4g+3 of each of two blocks) is exactly the B operand of O^T = V_hat^T P^T with
-//           those 8 tokens as its k-slots; the A operand is the dequantized V of the two
-//           blocks, 16 bytes per lane and dimension tile.  O^T accumulates in fp32; the parts'
-//           partials are summed in part order by the last part to finish, and leave as BF16,
-//           four dimensions of one row per lane.
-// Both passes stream stages of four blocks whose K (and dequantized V) the workgroup's four
-// wavefronts load once and share through LDS, one barrier per stage.
-// Rows are head-major (row r: head r / S, token r % S) as in the other kernels.  Row r sees
-// keys j <= T - S + r % S (the eager mask); T >= S is the caller's contract (the S new tokens
-// are part of the context), and a row that sees no key outputs 0.  The page ids of the
-// workgroup's blocks are staged in LDS, kPrefillWindow at a time.  Measured steps (2048 x 8192,
-// 12/2/128 and 14/2/64, both passes): 451 / 324 us with 16 rows per wavefront and V dequantized
-// per stage into LDS by the workgroup; scalar branches for the unmasked stages 442 / 281;
-// two row tiles in pass 1 382 / 263; two in pass 2 350 / 235; V dequantized by pass 1 and
-// MFMA results in VGPRs 332 / 218; 16-byte part slots and key parts per launch size 303 / 196;
-// each stage's K and V loaded once per workgroup and shared through LDS 284 / 182; stages of
-// four blocks, products issued by phase 271 / 173; v_max3 for the stage max and register
-// budgets held per pass 265 / 171; constant block indices in the loads and 1/L folded into
-// the exponent 258 / 167 (worst rel-L2 per 64-row block against eager 1.8e-4 -> 2.3e-4); pass
-// 2's statistics loads eight parts at a time 253 / 160.
-constexpr int kPrefillRows = 16;   // query rows per MFMA row tile
-constexpr int kPass1Waves = 4;     // wavefronts per workgroup, pass 1
-constexpr int kPass2Waves = 4;     // and pass 2
-constexpr int prefill_waves(bool OUT) { return OUT ? kPass2Waves : kPass1Waves; }
-constexpr int kPrefillWindow = 256;   // page ids staged in LDS per round
-constexpr int kStageBlocks = 4;      // page blocks per stage (a multiple of 2 dividing the window)
-// Pass 1: row tiles per wavefront (each K operand it loads serves this many tiles; 2048 x 8192,
-// pass 1 with one tile 158 / 93 us (12/2/128 / 14/2/64), with two 101 / 77 us)
-constexpr int kPass1Tiles = 2;
-// Pass 2: row tiles per wavefront, and the rows of a workgroup (a row group: its part slots,
-// its counter)
-constexpr int kPass2Tiles = 2;
-constexpr int kPass2Rows = kPass2Tiles * kPrefillRows * kPass2Waves;
-// Both passes split each row group's keys in parts, one workgroup each (pass 2 merges pass 1's
-// (max, sum) in part order; the last pass-2 part to finish sums the parts' outputs), as many
-// as bring the launch to about this many workgroups, at most kPrefillMaxParts and none under
-// 8 blocks.  Pass 1: 2048 x 8192 in 8 parts (12/2/128: 101 us, 16 parts 108 us; 14/2/64: 74 us,
-// 11 parts 83 us, 6 parts 80 us);
-// pass 2: one round, two wavefronts per SIMD for head_dim 128 and three for 64 (2048 x 8192: 2
-// parts 12/2/128, 3 parts 14/2/64).
-constexpr int pass1_workgroups(int D) { return D == 128 ? 1536 : 1792; }
-constexpr int pass2_workgroups(int D) { return D == 128 ? 512 : 768; }
-constexpr int kPrefillMaxParts = 64;
-// pass 2: the last part to finish adds every part's slot of its row group
-constexpr int kPrefillMaxParts2 = 8;
-
-// Resident wavefronts per SIMD the register budget is held to: pass 1 four (at most 128
-// VGPRs), pass 2 three for head_dim 64 (168) and two for 128 (its 64 fp32 accumulators per lane).
-constexpr int prefill_waves_per_simd(int D, bool OUT) { return !OUT ? 4 : D == 64 ? 3 : 2; }
-
-// Pass 2's parts of row group k (0-based within its head) when they follow its key count:
-// the group's last row sees keys up to T - S + min(S, rows * (k + 1)) - 1, in blocks of 16, cut
-// into parts of at most kstar blocks.  The host plans with T = max_seq_len; the kernel maps
-// its workgroups with the same arguments, so both agree on the grid.
-__host__ __device__ inline int pass2_group_parts(int k, int S, int T, int rows, int kstar) {
-  const int keys = T - S + min(S, rows * (k + 1));
-  const int blocks = keys > 0 ? (keys + kBlock - 1) / kBlock : 0;
-  return max(1, (blocks + kstar - 1) / kstar);
-}
-
-template <int D, bool OUT>
-__global__ __launch_bounds__(64 * prefill_waves(OUT)) __attribute__((amdgpu_waves_per_eu(prefill_waves_per_simd(D, OUT))))
-void prefill_kernel(AttnArgs a) {
-  // row tiles of 16 rows per wavefront (two in both passes: each K operand a wavefront reads
-  // serves 32 rows)
-  constexpr int KK = D / 32, DT = D / 16, NT = OUT ? kPass2Tiles : kPass1Tiles, ROWS = NT * 16;
-  constexpr int W = prefill_waves(OUT);
-  constexpr int DTW = DT / W;  // pass 1: dimension tiles of V each wavefront dequantizes
-  static_assert(OUT || DTW * W == DT, "the wavefronts share the dimension tiles evenly");
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  __shared__ int lpb[kPrefillWindow];
-  __shared__ int s_kend;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, n = lane & 15;
-  const int kvh = blockIdx.y, zb = blockIdx.z, b = zb % a.B, layer = zb / a.B;
-  const int T = seq_len_of(a, b);
-  const int grp = zb * a.KV + kvh;
-  // the keys of a row group are split in parts, one workgroup each: a.pf_split in pass 1,
-  // a.pf_parts in pass 2
-  int nparts = OUT ? a.pf_parts : a.pf_split;
-  int split = (int)(blockIdx.x % nparts);
-  int rgi = (int)(blockIdx.x / nparts);
-  if (OUT && a.pf_kstar > 0) {  // parts per row group by its key count: head h, then group k
-    const int rgph = a.S / kPass2Rows;
-    const int h = (int)blockIdx.x / a.pf_wh;
-    int off = (int)blockIdx.x - h * a.pf_wh, k = 0;
-    for (; k < rgph - 1; ++k) {
-      const int pk = pass2_group_parts(k, a.S, a.max_seq_len, kPass2Rows, a.pf_kstar);
-      if (off < pk) break;
-      off -= pk;
-    }
-    nparts = pass2_group_parts(k, a.S, a.max_seq_len, kPass2Rows, a.pf_kstar);
-    split = off;
-    rgi = h * rgph + k;
-  }
-  const int row0 = (rgi * W + wave) * ROWS;
-
-  // this lane's rows (row tile nt: row row0 + nt*16 + n): q operand and last visible key
-  bf16x8 qop[NT][KK];
-  int lim[NT];
-  bool rv[NT];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int r = row0 + nt * 16 + n;
-    rv[nt] = r < a.R;
-    const int hl = rv[nt] ? r / a.S : 0, si = rv[nt] ? r % a.S : 0;
-    const uint16_t* qp = a.q + layer * a.q_ls + b * a.q_sb + (int64_t)(kvh * a.G + hl) * a.q_sh + si * a.q_ss + g * 8;
-#pragma unroll
-    for (int kk = 0; kk < KK; ++kk) qop[nt][kk] = rv[nt] ? load_bf16x8(qp + kk * 32) : zero_bf16x8();
-    lim[nt] = rv[nt] ? min(T - 1, T - a.S + si) : -1;
-  }
-  // blocks this wavefront streams (keys 0 .. max lim) and the smallest lim of its rows (every
-  // key up to it is seen by every row: the blocks below nfull need no mask).  Both are
-  // wave-uniform and kept in scalar registers, so that every branch on them below is a
-  // scalar branch rather than a change of the execution mask.
-  int kend = 0, kmin = INT_MAX;
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    kend = max(kend, lim[nt] + 1);
-    kmin = min(kmin, rv[nt] ? lim[nt] : INT_MAX);
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    kend = max(kend, __shfl_xor(kend, off));
-    kmin = min(kmin, __shfl_xor(kmin, off));
-  }
-  const int nblk = __builtin_amdgcn_readfirstlane((kend + kBlock - 1) >> 4);
-  const int nfull = __builtin_amdgcn_readfirstlane(kmin == INT_MAX ? 0 : max(0, (kmin + 1) >> 4));
-  if (tid == 0) s_kend = 0;
-  __syncthreads();
-  if (lane == 0) atomicMax(&s_kend, nblk);
-  __syncthreads();
-  const int nblk_wg = __builtin_amdgcn_readfirstlane(s_kend);
-
-  // page addressing: a page id's base is scalar (this layer and KV head), the lane's offset a
-  // 32-bit vector offset
-  const uint16_t* klayer = a.k_pages + layer * a.k_ls + (int64_t)kvh * (kBlock * D);
-  const uint8_t* vlayer = a.v_pages + layer * a.v_ls + (int64_t)kvh * (D * kBlock);
-  const float* slayer = a.v_scales + layer * a.s_ls + (int64_t)kvh * kBlock;
-  const int64_t kpage = (int64_t)a.KV * (kBlock * D);  // K elements, V bytes per page id
-  const int64_t spage = (int64_t)a.KV * kBlock;        // scales per page id
-  const unsigned koff = (unsigned)lane * 8u;
-  const unsigned voff = (unsigned)((wave * DTW * 16 + n) * kBlock + 4 * g);
-  const int* btrow = a.block_table + (int64_t)b * a.max_blocks;
-  float2* st = a.stats + (int64_t)grp * a.R * a.pf_split;  // row r, pass-1 part k: st[r * a.pf_split + k]
-  // this workgroup's key blocks: part `split` of [0, nblk_wg)
-  const int part = (((nblk_wg + nparts - 1) / nparts) + kStageBlocks - 1) & ~(kStageBlocks - 1);  // whole stages
-  const int blo = min(nblk_wg, split * part);
-  const int bhi = min(nblk_wg, blo + part);
-
-  // Scores in the eager units: bf16(bf16(x) / sqrt(D)).  For head_dim 64 the divisor is 8 and
-  // bf16(x) * 0.125 is exact, so the scores are kept as bf16(x) -- one rounding -- and the
-  // factor 0.125 goes into the row max (exact) and into the exponent's coefficient
-  // (kLog2e * 0.125 is exact, so fma(bf16(x), kLog2e * 0.125, c) is bit for bit
-  // fma(bf16(x) * 0.125, kLog2e, c)).
-  constexpr float kUnit = D == 64 ? 0.125f : 1.0f;
-  constexpr float kExpCoef = kLog2e * kUnit;
-  const float csc = a.inv_sqrt_d;
-  auto eager4 = [&](const f32x4& s, float* y) {
-    if constexpr (D == 64) {
-      const uint32_t r01 = pack_bf16x2(s[0], s[1]), r23 = pack_bf16x2(s[2], s[3]);
-      y[0] = bf16_lo(r01);
-      y[1] = bf16_hi(r01);
-      y[2] = bf16_lo(r23);
-      y[3] = bf16_hi(r23);
-    } else {
-      float t[4];
-      round_scaled4(s[0], s[1], s[2], s[3], csc, t);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) y[i] = t[i];
-    }
-  };
-
-  float m_run[NT], l_run[NT];   // pass 1: running max and sum
-  float nml[NT];                // pass 2: -M log2 e - log2 L per row
-  f32x4 acc[DT][NT];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    m_run[nt] = -INFINITY;
-    l_run[nt] = 0.0f;
-    nml[nt] = 0.0f;
-    if (OUT && rv[nt]) {
-      // (M, L) of the row: its parts merged in part order
-      const float2* sr = st + (int64_t)(row0 + nt * 16 + n) * a.pf_split;
-      // eight parts' loads in flight at a time, merged in part order
-      float m = -INFINITY, l = 0.0f;
-      for (int k0 = 0; k0 < a.pf_split; k0 += 8) {
-        float2 v[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = k0 + i < a.pf_split ? sr[k0 + i] : make_float2(-INFINITY, 0.0f);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          if (k0 + i == 0) {
-            m = v[0].x;
-            l = v[0].y;
-          } else {
-            merge_fast(m, l, v[i].x, v[i].y);
-          }
-        }
-      }
-      if (l > 0.0f) {
-        // p = exp(s - M) / L as one exp2: 2^(s log2 e - M log2 e - log2 L) (v_log_f32 is within
-        // 1 ulp; |log2 L| <= log2 T, so p moves by ~1e-6 relative, far below its BF16 step)
-        nml[nt] = -m * kLog2e - __builtin_amdgcn_logf(l);
-      }
-    }
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) acc[dt][nt] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-  }
-
-  // A stage is kStageBlocks = 4 consecutive blocks u = 0..3.  Its K operands (4 x KK chunks of
-  // 1 KiB: block u, 32-dimension slice kk, in the lane order of the MFMA's A operand) and, for
-  // pass 2, its dequantized V operand (2 x DT chunks of 1 KiB: pair h of blocks, dimension tile
-  // dt, written by pass 1) are the same for every row, so the workgroup loads each chunk once
-  // and shares it through LDS: wavefront w loads chunks w, w + W, ... of stage s + 2 into
-  // registers while the workgroup computes stage s, and writes them to the LDS buffer of stage
-  // s right after the barrier of stage s + 1.  One barrier per stage publishes the stage and
-  // frees the other buffer.  Within a stage the q.k^T products of all four blocks go out
-  // first, then the scores, then the p.V products: the MFMA unit has independent work while
-  // the VALU rounds.
-  constexpr int SB = kStageBlocks;
-  constexpr int NKC = SB * KK, NC = NKC + (OUT ? (SB / 2) * DT : 0), CPW = NC / W;
-  static_assert(CPW * W == NC && NKC % W == 0, "the wavefronts share the chunks evenly");
-  __shared__ uint4 ring[2][NC * 64];
-  const uint4* vh_grp = a.vhat + (int64_t)grp * a.vh_stages * (DT * 64) + lane;
-  for (int w0 = blo; w0 < bhi; w0 += kPrefillWindow) {  // workgroup-uniform
-    const int wn = min(kPrefillWindow, bhi - w0);
-    __syncthreads();  // the previous window's page ids are no longer read
-    for (int j = tid; j < wn; j += 64 * W) {
-      const int pb = btrow[w0 + j];
-      lpb[j] = (pb >= 0 && pb < a.num_blocks) ? pb : -1;
-    }
-    __syncthreads();
-    const int jn = max(0, min(nblk - w0, wn));  // this wavefront's blocks in the window
-    const int nst = (wn + SB - 1) / SB;         // the workgroup's stages in the window
-    // page id of block jb of the window (jb < wn; the same word in every lane)
-    auto page = [&](int jb) { return __builtin_amdgcn_readfirstlane(lpb[jb]); };
-    uint4 stg[CPW];  // this wavefront's chunks of the next stage
-    auto fetch = [&](int s4) {
-#pragma unroll
-      for (int j = 0; j < CPW; ++j) {
-        const int c = j * W + wave;
-        if (j < NKC / W) {  // a K chunk: block u, slice kk; past the window, page 0 (never used)
-          // u is a constant when every wavefront's chunk j falls in the same block
-          const int u = KK % W == 0 ? (j * W) / KK : c / KK, kk = c - u * KK;
-          const int jb = SB * s4 + u;
-          const int pb = __builtin_amdgcn_readfirstlane(lpb[min(jb, kPrefillWindow - 1)]);
-          const int64_t pg = jb < wn ? max(pb, 0) : 0;
-          stg[j] = load_stream16(klayer + pg * kpage + (koff + kk * 512u));
-        } else {            // a dequantized V chunk: pair h, dimension tile dt
-          const int h = DT % W == 0 ? (j * W - NKC) / DT : (c - NKC) / DT, dt = (c - NKC) - h * DT;
-          const int sg = min((w0 >> 1) + (SB / 2) * s4 + h, a.vh_stages - 1);
-          stg[j] = vh_grp[(int64_t)sg * (DT * 64) + dt * 64];
-        }
-      }
-    };
-    auto stash = [&](int s4) {
-#pragma unroll
-      for (int j = 0; j < CPW; ++j) ring[s4 & 1][(j * W + wave) * 64 + lane] = stg[j];
-    };
-    auto compute_stage = [&](int s4, const uint4* sb) {
-      const int jb0 = SB * s4, jg0 = w0 + jb0;  // window and global block of u = 0
-      int pb[SB];
-#pragma unroll
-      for (int u = 0; u < SB; ++u) pb[u] = jb0 + u < jn ? page(jb0 + u) : -1;
-      // scalar: every key of the stage exists, is valid and is seen by every row
-      bool full = jg0 + SB <= nfull && jb0 + SB <= jn;
-#pragma unroll
-      for (int u = 0; u < SB; ++u) full = full && pb[u] >= 0;
-      // q.k^T of the stage's blocks, all issued before any score is rounded
-      f32x4 sacc[SB][NT];
-#pragma unroll
-      for (int kk = 0; kk < KK; ++kk)
-#pragma unroll
-        for (int u = 0; u < SB; ++u) {
-          const bf16x8 kop = __builtin_bit_cast(bf16x8, sb[(u * KK + kk) * 64 + lane]);
-#pragma unroll
-          for (int nt = 0; nt < NT; ++nt)
-            sacc[u][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kop, qop[nt][kk], kk == 0 ? (f32x4){0.0f, 0.0f, 0.0f, 0.0f} : sacc[u][nt], 0, 0, 0);
-        }
-      float y[NT][4 * SB];  // the stage's scores (in units of kUnit): block u in 4u .. 4u+3
-#pragma unroll
-      for (int u = 0; u < SB; ++u)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) eager4(sacc[u][nt], y[nt] + 4 * u);
-      if (!full) {
-#pragma unroll
-        for (int u = 0; u < SB; ++u) {
-          const int t0 = (jg0 + u) * kBlock + 4 * g;
-          const bool blk_ok = pb[u] >= 0;  // -1 also for a block past this wavefront's
-#pragma unroll
-          for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) y[nt][4 * u + i] = (blk_ok && t0 + i <= lim[nt]) ? y[nt][4 * u + i] : -INFINITY;
-        }
-      }
-      if constexpr (!OUT) {
-        // Online (max, sum) per lane, one update per stage: the max of the stage's scores first,
-        // then the running sum rescaled once by exp2((m_old - m_new) log2 e), which is exactly 1
-        // while the max stays (the one-FMA form exp2(m_old log2 e - RN(m_new log2 e)) is off by
-        // the product's rounding on every update, and L drifted by ~1e-5 at T = 8192: rel-L2
-        // 7e-4 against eager).  A lane sums at most T/32 terms of at most 1 each, so the plain
-        // fp32 sum is within ~1e-5 relative of the exact one.  A stage without masked keys has
-        // a finite max, and exp2(-inf) = 0 covers the first update.
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-          const float* yt = y[nt];
-          static_assert(SB == 4, "the max below covers 16 scores");
-          const float m0 = max3f(yt[0], yt[1], yt[2]), m1 = max3f(yt[3], yt[4], yt[5]), m2 = max3f(yt[6], yt[7], yt[8]);
-          const float m3 = max3f(yt[9], yt[10], yt[11]), m4 = max3f(yt[12], yt[13], yt[14]);
-          const float mt = max3f(max3f(m0, m1, m2), max3f(m3, m4, yt[15]), -INFINITY) * kUnit;
-          if (full || mt != -INFINITY) {
-#pragma clang fp contract(off)
-            const float mn = fmaxf(m_run[nt], mt), nm = -mn * kLog2e;
-            const float f = __builtin_amdgcn_exp2f((m_run[nt] - mn) * kLog2e);
-            float e[4 * SB];
-#pragma unroll
-            for (int i = 0; i < 4 * SB; ++i) e[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(yt[i], kExpCoef, nm));
-            float xs[SB];
-#pragma unroll
-            for (int u = 0; u < SB; ++u) xs[u] = (e[4 * u] + e[4 * u + 1]) + (e[4 * u + 2] + e[4 * u + 3]);
-            l_run[nt] = l_run[nt] * f + ((xs[0] + xs[1]) + (xs[2] + xs[3]));
-            m_run[nt] = mn;
-          }
-        }
-      } else {
-        // p for each pair h of blocks: the B operand of one p.V product (tokens 4g..4g+3 of the
-        // pair's first block, then of its second)
-        bf16x8 pop[SB / 2][NT];
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-          for (int h = 0; h < SB / 2; ++h) {
-            uint32_t pw[4];
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-              const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(y[nt][8 * h + 2 * w], kExpCoef, nml[nt]));
-              const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(y[nt][8 * h + 2 * w + 1], kExpCoef, nml[nt]));
-              pw[w] = pack_bf16x2(p0, p1);
-            }
-            pop[h][nt] = __builtin_bit_cast(bf16x8, make_uint4(pw[0], pw[1], pw[2], pw[3]));
-          }
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-          for (int h = 0; h < SB / 2; ++h) {
-            const bf16x8 vop = __builtin_bit_cast(bf16x8, sb[(NKC + h * DT + dt) * 64 + lane]);
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) acc[dt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop, pop[h][nt], acc[dt][nt], 0, 0, 0);
-          }
-      }
-    };
-    fetch(0);
-    stash(0);
-    fetch(1);
-    for (int ss = 0; ss < nst; ++ss) {  // workgroup-uniform
-      // stage ss is in LDS for every wavefront, and every wavefront is done with stage ss - 1
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-      __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-      stash(ss + 1);  // into the buffer of stage ss - 1
-      fetch(ss + 2);
-      if (SB * ss < jn) compute_stage(ss, ring[ss & 1]);  // scalar: the stage has keys this wavefront's rows see
-    }
-  }
-
-  if constexpr (!OUT) {
-    // Pass 2's V operand: stage sg of the group (blocks 2sg, 2sg+1) is dequantized by this
-    // launch's workgroup sg mod gridDim.x, one dimension tile group per wavefront, as
-    // bf16(fp32(code) * scale).  Codes and scales of tokens that are not in the sequence (past
-    // T, invalid or absent blocks) become 0, so that no NaN pattern of an unwritten slot reaches
-    // the MFMA.
-    const int nbk = (T + kBlock - 1) / kBlock;
-    for (int sg = (int)blockIdx.x; sg < (nbk + 1) >> 1; sg += (int)gridDim.x) {
-      uint32_t w[2][DTW];
-      float4 sc[2];
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int jb = 2 * sg + u;
-        int pb = jb < nbk ? btrow[jb] : -1;
-        pb = (pb >= 0 && pb < a.num_blocks) ? pb : -1;
-        const int64_t pg = max(pb, 0);
-        const uint8_t* vp = vlayer + pg * kpage;
-#pragma unroll
-        for (int dtl = 0; dtl < DTW; ++dtl) w[u][dtl] = *reinterpret_cast<const uint32_t*>(vp + (voff + dtl * 16u * kBlock));
-        sc[u] = *reinterpret_cast<const float4*>(slayer + pg * spage + 4 * g);
-        const int t0 = jb * kBlock + 4 * g;
-        const int nv = pb >= 0 ? min(max(T - t0, 0), 4) : 0;
-        const uint32_t mask = nv >= 4 ? 0xFFFFFFFFu : (1u << (8 * nv)) - 1u;
-#pragma unroll
-        for (int dtl = 0; dtl < DTW; ++dtl) w[u][dtl] &= mask;
-        sc[u].x = nv > 0 ? sc[u].x : 0.0f;
-        sc[u].y = nv > 1 ? sc[u].y : 0.0f;
-        sc[u].z = nv > 2 ? sc[u].z : 0.0f;
-        sc[u].w = nv > 3 ? sc[u].w : 0.0f;
-      }
-      uint4* dst = a.vhat + ((int64_t)grp * a.vh_stages + sg) * (DT * 64) + lane;
-#pragma unroll
-      for (int dtl = 0; dtl < DTW; ++dtl) {
-        const f32x2 f01 = __builtin_amdgcn_cvt_pk_f32_fp8(w[0][dtl], false);
-        const f32x2 f23 = __builtin_amdgcn_cvt_pk_f32_fp8(w[0][dtl], true);
-        const f32x2 f45 = __builtin_amdgcn_cvt_pk_f32_fp8(w[1][dtl], false);
-        const f32x2 f67 = __builtin_amdgcn_cvt_pk_f32_fp8(w[1][dtl], true);
-        dst[(wave * DTW + dtl) * 64] =
-            make_uint4(pack_bf16x2(f01.x * sc[0].x, f01.y * sc[0].y), pack_bf16x2(f23.x * sc[0].z, f23.y * sc[0].w),
-                       pack_bf16x2(f45.x * sc[1].x, f45.y * sc[1].y), pack_bf16x2(f67.x * sc[1].z, f67.y * sc[1].w));
-      }
-    }
-  }
-
-  if constexpr (!OUT) {
-    // (max, sum) of each row over the four lane groups, in a fixed order
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      float m = m_run[nt], l = l_run[nt];
-      merge_lanes<16>(m, l);
-      merge_lanes<32>(m, l);
-      if (g == 0 && rv[nt]) st[(int64_t)(row0 + nt * 16 + n) * a.pf_split + split] = make_float2(m, l);
-    }
-  } else {
-    // lane (g, n) holds O^T[dims dt*16 + 4g .. +3][row nt*16 + n] of this part's keys
-    bool write = true;
-    if (nparts > 1) {  // workgroup-uniform
-      // Every part writes its fp32 partial to its slot (device-scope stores), waits for them,
-      // and counts itself in the row group's counter -- a (call tag, count) word in the sync
-      // area, read as 0 when it carries another call's tag.  The part that completes the count
-      // sums the slots in part order (its own from registers), writes the output and zeroes the
-      // counter.  Nobody waits for anybody: the order of arrival changes who sums, not the sum.
-      const int nrg = (a.R + kPass2Rows - 1) / kPass2Rows;
-      constexpr int slot_b = kPass2Rows * D * 4;  // bytes per part slot
-      // the row group's slots, written and read with 16-byte device-scope (sc1) accesses
-      const __amdgpu_buffer_rsrc_t srs = __builtin_amdgcn_make_buffer_rsrc(
-          a.partial + ((int64_t)grp * nrg + rgi) * a.pf_parts * (slot_b / 4), (short)0, nparts * slot_b, 0x00020000);
-      // lane (g, n): row wave*ROWS + nt*16 + n, dimensions dt*16 + 4g .. +3
-      const int lofs = ((wave * ROWS + n) * D + 4 * g) * 4;
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, acc[dt][nt]), srs,
-                                                 split * slot_b + lofs + (nt * 16 * D + dt * 16) * 4, 0, 16);
-      __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      SDV_VMCNT0();
-      __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      __syncthreads();
-      __shared__ int s_last;
-      if (tid == 0) {
-        uint64_t* ctr = reinterpret_cast<uint64_t*>(a.sync) + kSyncHeadBytes / 8 + (int64_t)grp * nrg + rgi;
-        uint64_t old = load_dev_u64(ctr);
-        uint32_t mine = 0;
-        for (;;) {  // compare-and-swap against the other parts of this row group only
-          const uint32_t cnt = (uint32_t)(old >> 32) == a.tag ? (uint32_t)old : 0u;
-          const uint64_t nw = ((uint64_t)a.tag << 32) | (cnt + 1u);
-          const uint64_t prev = atomicCAS(reinterpret_cast<unsigned long long*>(ctr), (unsigned long long)old,
-                                          (unsigned long long)nw);
-          if (prev == old) {
-            mine = cnt + 1u;
-            break;
-          }
-          old = prev;
-        }
-        const bool last = mine == (uint32_t)nparts;
-        if (last) store_dev_u64(ctr, 0);
-        s_last = last;
-      }
-      __syncthreads();
-      write = s_last;
-      if (write) {
-        // the parts' sum in part order, each part's slot loaded whole before it is added
-        f32x4 sum[DT][NT];
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-          for (int dt = 0; dt < DT; ++dt) sum[dt][nt] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-        for (int k = 0; k < nparts; ++k) {  // workgroup-uniform
-          f32x4 v[DT][NT];
-          if (k == split) {
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-              for (int dt = 0; dt < DT; ++dt) v[dt][nt] = acc[dt][nt];
-          } else {
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-              for (int dt = 0; dt < DT; ++dt)
-                v[dt][nt] = __builtin_bit_cast(
-                    f32x4, __builtin_amdgcn_raw_buffer_load_b128(srs, k * slot_b + lofs + (nt * 16 * D + dt * 16) * 4, 0, 16));
-          }
-#pragma unroll
-          for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) sum[dt][nt] += v[dt][nt];
-        }
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-          for (int dt = 0; dt < DT; ++dt) acc[dt][nt] = sum[dt][nt];
-      }
-    }
-    if (write) {
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        if (!rv[nt]) continue;
-        const int r = row0 + nt * 16 + n, hl = r / a.S, si = r % a.S;
-        uint16_t* op = a.out + layer * a.q_ls + b * a.q_sb + (int64_t)(kvh * a.G + hl) * a.q_sh + si * a.q_ss + 4 * g;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-          *reinterpret_cast<uint2*>(op + dt * 16) =
-              make_uint2(pack_bf16x2(acc[dt][nt][0], acc[dt][nt][1]), pack_bf16x2(acc[dt][nt][2], acc[dt][nt][3]));
-      }
-    }
-  }
-}
+}  // namespace sdv
+#include "sdv_prefill.h"
+namespace sdv {
 
 // ---------------------------------------------------------------------------- group
 // Many (layer*batch, KV head) groups of one row tile each -- decode and short verify over many
@@ -2538,13 +2010,74 @@ struct Plan {
   int64_t groups;
   bool group;                                     // group_kernel serves the call (many one-tile groups)
   int tpad;                                       // group_kernel: scratch row length (tokens)
-  int pf_parts;                                   // prefill pass 2: key parts per row group
-  int pf_split;                                   // prefill pass 1: key parts per row group
-  int pf_kstar, pf_wh;                            // prefill pass 2: parts by key count (0: uniform)
+  int pf_nrg, pf_w1, pf_w2, pf_min1, pf_min2;     // prefill: see AttnArgs
+  int pf_split, pf_slots, pf_dense;
   size_t off_vhat;                                // prefill: dequantized V (pass 1 -> pass 2)
   int vh_stages;                                  // prefill: two-block stages per group
   size_t total;                                   // bytes for every layout the call may take
 };
+
+// The prefill part of a plan.  The workspace holds the (max, sum) of each row and pass-1 segment,
+// fp32 part slots and V dequantized once.  Its size follows a fixed rule: statistics for as many
+// key parts as bring 128-row workgroups to about 1,536 / 1,792 (head_dim 128 / 64), slots for as
+// many as bring them to 512 / 768, with S a multiple of 128 the fewest blocks per part that stay
+// within that; the launches' split is chosen to fit what it gives.
+static void plan_prefill(int64_t groups, int R, int S, int G, int D, int T, Plan* p) {
+  const int nbk = (T + kBlock - 1) / kBlock;
+  constexpr int kSizeRows = 128, kSizeStage = 4;  // rows and blocks of the size rule
+  const int max_parts = std::min(64, std::max(1, nbk / 8));
+  const int64_t nrg128 = (R + kSizeRows - 1) / kSizeRows;
+  p->pf_split = (int)std::max<int64_t>(1, std::min<int64_t>(max_parts, (D == 128 ? 1536 : 1792) / (groups * nrg128)));
+  const int64_t budget = D == 128 ? 512 : 768;
+  int64_t parts = groups * nrg128 <= (int64_t)(kSyncStatsBytes / 8)
+                      ? std::max<int64_t>(1, std::min<int64_t>(std::min(max_parts, 8), budget / (groups * nrg128)))
+                      : 1;
+  if (parts > 1 && S % kSizeRows == 0) {
+    const int rgph = S / kSizeRows;
+    for (int kstar = kSizeStage; kstar < nbk + kSizeStage; kstar += kSizeStage) {
+      int64_t wh = 0, pmax = 0;
+      for (int k = 0; k < rgph; ++k) {
+        const int keys = T - S + std::min(S, kSizeRows * (k + 1));
+        const int64_t pk = std::max(1, ((keys > 0 ? (keys + kBlock - 1) / kBlock : 0) + kstar - 1) / kstar);
+        wh += pk;
+        pmax = std::max(pmax, pk);
+      }
+      if (groups * G * wh <= budget && pmax <= 8) {
+        if (pmax > 1) parts = pmax;
+        break;
+      }
+    }
+  }
+  const size_t stats = round_up((size_t)(groups * R * 8 * p->pf_split), 256);
+  const size_t slots = parts > 1 ? round_up((size_t)(groups * nrg128 * parts * kSizeRows * D * 4), 256) : 0;
+  p->off_partial = p->off_stats + stats;
+  p->vh_stages = (nbk + 1) / 2;
+  p->off_vhat = p->off_partial + slots;
+  p->total = p->off_vhat + (size_t)groups * p->vh_stages * (D / 16) * 1024;
+
+  p->pf_nrg = (R + kPfRows - 1) / kPfRows;
+  const int64_t nrg = groups * p->pf_nrg;  // row groups of the call
+  int64_t stages = 0;
+  for (int i = 0; i < p->pf_nrg; ++i) stages += kPfSegStages + pf_stages(i, S, G, T);
+  const int64_t U = stages * groups;
+  const int64_t slot_b = (int64_t)kPfRows * D * 4;
+  p->pf_slots = (int)(slots / slot_b);
+  const int64_t have = p->pf_slots + (int64_t)(kSyncPartBytes - kPfDescBytes) / slot_b;
+  const int64_t cap1 = kPfCus * pf_wgs_per_cu(D, false), cap2 = kPfCus * pf_wgs_per_cu(D, true);
+  p->pf_min1 = p->pf_min2 = kPfMinStages;
+  // A range's partial row groups need a slot each: W + nrg in all, and 2 per workgroup at most
+  const int64_t w2 = std::min({cap2, std::max(have / 2, have - nrg), (U + kPfMinStages - 1) / kPfMinStages});
+  if (U >= (1 << 30) || nbk >= (1 << 22) || nrg > kPfMaxGroups || w2 < std::min(nrg, cap2)) return;  // whole row groups
+  p->pf_w2 = (int)w2;
+  p->pf_dense = w2 + nrg <= have;
+  // pass 1: the ranges that cut a row group of ns stages, at most (ns - 2) / per + 2, fit its
+  // statistics
+  const int ns = pf_stages(p->pf_nrg - 1, S, G, T);
+  if (p->pf_split >= 2) {
+    p->pf_w1 = (int)std::min(cap1, (U + kPfMinStages - 1) / kPfMinStages);
+    p->pf_min1 = std::max(p->pf_min1, (ns - 1 + p->pf_split - 2) / (p->pf_split - 1));
+  }
+}
 
 static bool make_plan(int L, int B, int H, int KV, int S, int D, int max_seq_len, Plan* p) {
   if (L <= 0 || B <= 0 || H <= 0 || KV <= 0 || S <= 0 || max_seq_len <= 0) return false;
@@ -2582,61 +2115,14 @@ static bool make_plan(int L, int B, int H, int KV, int S, int D, int max_seq_len
   p->groups = groups;
   p->group = false;
   p->tpad = 0;
-  p->pf_parts = 1;
-  p->pf_split = 1;
-  p->pf_kstar = 0;
-  p->pf_wh = 0;
+  p->pf_nrg = p->pf_w1 = p->pf_w2 = p->pf_min1 = p->pf_min2 = 0;
+  p->pf_split = p->pf_slots = p->pf_dense = 0;
   p->off_vhat = 0;
   p->vh_stages = 0;
-  if (p->n_row_groups > 1) {  // prefill kernels: the per-row (max, sum) of each key part
+  if (p->n_row_groups > 1) {  // prefill kernels
     p->off_scores = kSyncBytes;
     p->off_stats = kSyncBytes;
-    const int nbk = (max_seq_len + kBlock - 1) / kBlock;
-    const int max_parts = min(kPrefillMaxParts, max(1, nbk / 8));
-    const int64_t nrg1 = (R + kPass1Tiles * kPrefillRows * kPass1Waves - 1) / (kPass1Tiles * kPrefillRows * kPass1Waves);
-    p->pf_split = (int)std::max<int64_t>(1, std::min<int64_t>(max_parts, pass1_workgroups(D) / (groups * nrg1)));
-    const size_t stats = round_up((size_t)(groups * R * 8 * p->pf_split), 256);
-    p->off_partial = p->off_stats + stats;
-    // pass 2 splits the keys too when its counters (one per row group) fit the sync area's
-    // statistics region; its part slots follow the statistics
-    const int64_t nrg = (R + kPass2Rows - 1) / kPass2Rows;
-    p->pf_parts = groups * nrg <= (int64_t)(kSyncStatsBytes / 8)
-                      ? (int)std::max<int64_t>(1, std::min<int64_t>(std::min(max_parts, kPrefillMaxParts2), pass2_workgroups(D) / (groups * nrg)))
-                      : 1;
-    // With S a multiple of the pass's rows, the parts of each row group follow its key count
-    // (the offset-causal mask: the head's later rows see more keys): the fewest blocks per
-    // part that keep the launch within the same budget, so that the workgroups carry nearly
-    // equal work (2048 x 8192, 12/2/128: 504 workgroups of at most 216 blocks instead of 384 of
-    // up to 256, half of the CUs holding one)
-    p->pf_kstar = 0;
-    p->pf_wh = 0;
-    if (p->pf_parts > 1 && S % kPass2Rows == 0) {
-      const int rgph = S / kPass2Rows;
-      const int64_t heads = groups * G;  // (layer, sequence, query head): rgph row groups each
-      for (int kstar = kStageBlocks; kstar < nbk + kStageBlocks; kstar += kStageBlocks) {
-        int wh = 0, pmax = 0;
-        for (int k = 0; k < rgph; ++k) {
-          const int pk = pass2_group_parts(k, S, max_seq_len, kPass2Rows, kstar);
-          wh += pk;
-          pmax = std::max(pmax, pk);
-        }
-        if (heads * wh <= pass2_workgroups(D) && pmax <= kPrefillMaxParts2) {
-          if (pmax > 1) {
-            p->pf_kstar = kstar;
-            p->pf_wh = wh;
-            p->pf_parts = pmax;
-          }
-          break;
-        }
-      }
-    }
-    const size_t parts = p->pf_parts > 1
-                             ? round_up((size_t)(groups * nrg * p->pf_parts * kPass2Rows * D * 4), 256)
-                             : 0;
-    // pass 1 dequantizes V once for pass 2: D/16 x 1 KiB per stage of two blocks
-    p->vh_stages = (((max_seq_len + kBlock - 1) / kBlock) + 1) / 2;
-    p->off_vhat = p->off_partial + parts;
-    p->total = p->off_vhat + (size_t)groups * p->vh_stages * (D / 16) * 1024;
+    plan_prefill(groups, (int)R, S, G, D, max_seq_len, p);
     return true;
   }
   // the sync area [0, kSyncBytes) is shared by every layout and only the fused kernel uses it
@@ -2868,12 +2354,14 @@ template <int D>
 static bool launch_all(const AttnArgs& a, const Plan& p, int zdim, hipStream_t st, int phases) {
   if (p.n_row_groups > 1) {  // many query rows: the two prefill passes
     if (a.app_v) return false;
-    const dim3 grid((unsigned)((a.R + kPass2Rows - 1) / kPass2Rows), a.KV, zdim);
-    constexpr int rows1 = kPass1Tiles * 16 * kPass1Waves;  // pass 1 rows per workgroup
-    const dim3 grid1((unsigned)((a.R + rows1 - 1) / rows1) * a.pf_split, grid.y, grid.z),
-        grid2(a.pf_kstar > 0 ? (unsigned)(a.G * a.pf_wh) : grid.x * a.pf_parts, grid.y, grid.z);
-    if (phases & SDV_PHASE_QK) hipLaunchKernelGGL((prefill_kernel<D, false>), grid1, dim3(64 * kPass1Waves), 0, st, a);
-    if (phases & SDV_PHASE_PV) hipLaunchKernelGGL((prefill_kernel<D, true>), grid2, dim3(64 * kPass2Waves), 0, st, a);
+    const int layers = zdim / a.B;
+    const unsigned whole = (unsigned)(p.groups * p.pf_nrg);
+    if (phases & SDV_PHASE_QK)
+      hipLaunchKernelGGL((prefill_kernel<D, false>), dim3(p.pf_w1 ? p.pf_w1 : whole), dim3(64 * kPfWaves), 0, st, a, layers);
+    if (phases & SDV_PHASE_PV)
+      hipLaunchKernelGGL((prefill_kernel<D, true>), dim3(p.pf_w2 ? p.pf_w2 : whole), dim3(64 * kPfWaves), 0, st, a, layers);
+    if ((phases & SDV_PHASE_REDUCE) && p.pf_w2)
+      hipLaunchKernelGGL(prefill_reduce_kernel<D>, dim3(whole * kPfWaves), dim3(256), 0, st, a);
     return true;
   }
   if (phases == SDV_PHASE_ALL) {
@@ -3017,10 +2505,14 @@ static int attention(const void* q, const void* k_pages, const void* v_pages, co
   a.pv_chunk_tokens = p.pv_chunk_tokens;
   a.n_pv_chunks = p.n_pv_chunks;
   a.score_stride = p.score_stride;
-  a.pf_parts = p.pf_parts;
+  a.pf_nrg = p.pf_nrg;
+  a.pf_w1 = p.pf_w1;
+  a.pf_w2 = p.pf_w2;
+  a.pf_min1 = p.pf_min1;
+  a.pf_min2 = p.pf_min2;
   a.pf_split = p.pf_split;
-  a.pf_kstar = p.pf_kstar;
-  a.pf_wh = p.pf_wh;
+  a.pf_slots = p.pf_slots;
+  a.pf_dense = p.pf_dense;
   a.vhat = reinterpret_cast<uint4*>(ws + p.off_vhat);
   a.vh_stages = p.vh_stages;
   // RN(1/sqrt(D)): 1/sqrt(128) = 0.08838834764831845, 1/sqrt(64) = 0.125 exactly

@@ -199,3 +199,75 @@ def test_prefill_key_parts_repeat_and_replay(cuda_device, h, d, s):
         v_hat = oq.dequantize_kv_fp8(vc.cpu()[None], sc.cpu()[None], torch.bfloat16)
         want = oatt.eager_attention(q[b:b + 1].transpose(1, 2).cpu(), kc.cpu()[None], v_hat)
         assert_close(eager[0][b:b + 1].transpose(1, 2).cpu(), want, f"key parts b={b} T={t}")
+
+
+def test_prefill_many_row_groups_and_windows(cuda_device):
+    """260 row groups of one layer without part slots (130 sequences of 11 new rows): a workgroup
+    takes whole row groups, and at T = 33,000 (2,063 blocks) both passes stage the page ids in two
+    windows of 2,048.  The sequences share one sequence's pages; the first and the last are
+    checked."""
+    announce("prefill 130 sequences S=11 T=33000 (whole row groups, two page-id windows)")
+    b, h, kv, d, s, t = 130, 12, 2, 128, 11, 33000
+    g = wl.gen(750, cuda_device)
+    cache = PagedKVCache(kv, d, num_blocks=t // 16 + 3, device=cuda_device, seed=751, growable=False)
+    cache.prefill(0, torch.randn((t, kv, d), generator=g, device=cuda_device).to(torch.bfloat16),
+                  torch.randn((t, kv, d), generator=g, device=cuda_device).to(torch.bfloat16), [t])
+    q = torch.randn((b, s, h, d), generator=g, device=cuda_device).to(torch.bfloat16)
+    kp, vp, vs = cache.layer(0)
+    out = ops.paged_attention(q, kp, vp, vs, cache.block_table().expand(b, -1).contiguous(), None, t, q_token_major=True)
+    torch.cuda.synchronize()
+    kc, vc, sc = cache.gather(0, 0)
+    v_hat = oq.dequantize_kv_fp8(vc.cpu()[None], sc.cpu()[None], torch.bfloat16)
+    for i in (0, b - 1):
+        want = oatt.eager_attention(q[i:i + 1].transpose(1, 2).cpu(), kc.cpu()[None], v_hat)
+        assert_close(out[i:i + 1].transpose(1, 2).cpu(), want, f"sequence {i}")
+
+
+@pytest.mark.parametrize("h,d,s,t", [(12, 128, 300, 1500), (14, 64, 96, 900)])
+def test_prefill_late_maximum(cuda_device, h, d, s, t):
+    """Pass 1 takes its exponentials against the first stage's maximum and repeats a segment whose
+    sum overflows: scores that jump by far more than 88 in a later stage of the same segment."""
+    announce(f"prefill late maximum {h}/2/{d} S={s} T={t}")
+    g = wl.gen(760 + d, cuda_device)
+    cache = PagedKVCache(2, d, num_blocks=t // 16 + 3, device=cuda_device, seed=761, growable=False)
+    k = torch.randn((t, 2, d), generator=g, device=cuda_device)
+    for at in (200, 500, 777):   # past the first stage of a segment that begins at key 0, 256 or 512
+        k[at] = 4.0
+    v = torch.randn((t, 2, d), generator=g, device=cuda_device).to(torch.bfloat16)
+    q = (torch.randn((1, h, s, d), generator=g, device=cuda_device) * 0.25 + 4.0).to(torch.bfloat16)
+    cache.prefill(0, k.to(torch.bfloat16), v, [t])
+    kp, vp, vs = cache.layer(0)
+    out = ops.paged_attention(q, kp, vp, vs, cache.block_table(), cache.seq_lens_tensor(), t)
+    torch.cuda.synchronize()
+    kc, vc, sc = cache.gather(0, 0)
+    v_hat = oq.dequantize_kv_fp8(vc.cpu()[None], sc.cpu()[None], torch.bfloat16)
+    assert_close(out.cpu(), oatt.eager_attention(q.cpu(), kc.cpu()[None], v_hat), "late maximum")
+
+
+def test_prefill_skips_invalid_blocks(cuda_device):
+    """Block ids outside the pool are never read and their tokens are masked, in the pages every
+    row sees and on the diagonal: the output of the same call over a cache without those tokens."""
+    announce("prefill with invalid block ids")
+    h, kv, d, s, t = 12, 2, 128, 128, 1600
+    g = wl.gen(770, cuda_device)
+    k = torch.randn((t, kv, d), generator=g, device=cuda_device).to(torch.bfloat16)
+    v = torch.randn((t, kv, d), generator=g, device=cuda_device).to(torch.bfloat16)
+    cache = PagedKVCache(kv, d, num_blocks=t // 16 + 3, device=cuda_device, seed=771, growable=False)
+    cache.prefill(0, k, v, [t])
+    q = torch.randn((1, h, s, d), generator=g, device=cuda_device).to(torch.bfloat16)
+    kp, vp, vs = cache.layer(0)
+    holes = [3, 4, 40, 71, 99]   # 99: the last block, on the diagonal
+    table = cache.block_table().clone()
+    table[0, holes] = torch.tensor([-1, 1 << 20, -5, cache.alloc.num_blocks, -1], dtype=torch.int32, device=cuda_device)
+    out = ops.paged_attention(q, kp, vp, vs, table, cache.seq_lens_tensor(), t)
+    torch.cuda.synchronize()
+    kc, vc, sc = cache.gather(0, 0)
+    v_hat = oq.dequantize_kv_fp8(vc.cpu()[None], sc.cpu()[None], torch.bfloat16)
+    keep = torch.ones(t, dtype=torch.bool)
+    for j in holes:
+        keep[16 * j:16 * j + 16] = False
+    pos = torch.nonzero(keep).flatten()
+    for i in (0, 50, 127):       # row i sees the kept keys up to t - s + i
+        n = int((pos <= t - s + i).sum())
+        want = oatt.eager_attention(q[:, :, i:i + 1].cpu(), kc.cpu()[None][:, :, pos[:n]], v_hat[:, :, pos[:n]])
+        assert_close(out[:, :, i:i + 1].cpu(), want, f"row {i}")
