@@ -283,6 +283,19 @@ int sdv_paged_attention_noalloc(const void* q, const void* k_pages, const void* 
                                 int32_t q_len, int32_t head_dim, int32_t max_seq_len,
                                 int32_t q_token_major, void* out, void* stream);
 
+/*
+ * A contiguous v_fp8 cache into pages: k bf16 [batch][kv_heads][seq_len][head_dim], v_codes E4M3FN of
+ * the same shape, v_scales fp32 [batch][kv_heads][seq_len].  k_pages / v_pages / page_scales hold
+ * batch * ceil(seq_len/16) pages in the layout above, block b*ceil(seq_len/16) + j being tokens
+ * 16j.. of sequence b, and block_table int32 [batch][ceil(seq_len/16)] receives those block ids.
+ * Tokens past seq_len in a last block get K 0, code 0 and scale 1.  Alignment: k/k_pages 16 B,
+ * the rest 4 B.  For callers that hold the reference's cache tensors (model_self.py:778-800) and
+ * call its op over them (specdec/kernels/ops.py:67-76); no counterpart of its own.
+ */
+int sdv_pack_contiguous(const void* k, const void* v_codes, const float* v_scales, int32_t batch,
+                        int32_t kv_heads, int32_t seq_len, int32_t head_dim, void* k_pages, void* v_pages,
+                        float* page_scales, int32_t* block_table, void* stream);
+
 /* Elementwise fp32 -> E4M3FN (RNE, NaN beyond 464 / for Inf and NaN), device buffers. */
 int sdv_fp8_encode(const float* in, uint8_t* out, int64_t n, void* stream);
 

@@ -65,6 +65,7 @@ SIGNATURES = {
                                                   _P, _SZ, _P, _P, _P, _P, _I64, _I32, _P]),
     "sdv_paged_attention_noalloc": (ctypes.c_int, [_P, _P, _P, _P, _I32, _I64, _I64, _I64, _P, _I32, _P,
                                                    _I32, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _P, _P]),
+    "sdv_pack_contiguous": (ctypes.c_int, [_P, _P, _P, _I32, _I32, _I32, _I32, _P, _P, _P, _P, _P]),
     "sdv_fp8_encode": (ctypes.c_int, [_P, _P, _I64, _P]),
     "sdv_status_string": (ctypes.c_char_p, [ctypes.c_int]),
     "sdv_abi_version": (ctypes.c_int, []),

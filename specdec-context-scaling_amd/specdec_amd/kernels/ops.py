@@ -14,6 +14,7 @@ Operators
 ``attention``         the reference op's signature ``attention(q, k, v, backend)``
                       (ops.py:67-76) over a contiguous v_fp8 cache: k BF16 (B,KV,T,D) and
                       v given as the (payload, scale) pair the engine stores.
+                      One kernel packs the cache into pages first.
 ``fp8_encode``        elementwise fp32 -> E4M3FN on the device.
 """
 from __future__ import annotations
@@ -428,8 +429,50 @@ def attention(q: torch.Tensor, k: torch.Tensor, v, backend: str = "hip") -> torc
     _need(k, "k", (torch.bfloat16,), q.device, ndim=(4,))
     if payload.shape != k.shape or tuple(scale.shape) != tuple(k.shape[:3]) + (1,):
         _fail(f"v payload {tuple(payload.shape)} / scale {tuple(scale.shape)} do not match k {tuple(k.shape)}")
-    kp, vp, vs, bt, sl = pack_contiguous(k.contiguous(), payload.contiguous(), scale.contiguous())
-    return torch.ops.sdv.paged_attention(q.contiguous(), kp, vp, vs, bt, sl, k.shape[2])
+    return torch.ops.sdv.attention(q.contiguous(), k.contiguous(), payload.contiguous(), scale.contiguous())
+
+
+def _contiguous_attention(q: torch.Tensor, k: torch.Tensor, payload: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
+    """attention() over contiguous tensors: one kernel writes the cache into pages (the bytes
+    pack_contiguous gives), and the paged kernels run over them.  The pages, scales and block table
+    share one allocation."""
+    lib = _native.load()
+    _need(q, "q", (torch.bfloat16,), ndim=(4,))
+    dev = q.device
+    _need(k, "k", (torch.bfloat16,), dev, ndim=(4,))
+    if payload.element_size() != 1:
+        _fail(f"v payload must hold one byte per element (got {payload.dtype})")
+    _need(payload, "v payload", (payload.dtype,), dev)
+    _need(scale, "v scale", (torch.float32,), dev)
+    (B, H, S, D), (Bk, KV, T, Dk) = q.shape, k.shape
+    if Bk != B or Dk != D or KV <= 0 or H % KV:
+        _fail(f"q {tuple(q.shape)} does not match k {tuple(k.shape)}")
+    if T <= 0:
+        _fail(f"k {tuple(k.shape)} holds no tokens")
+    nbytes = attention_workspace_bytes(1, B, H, KV, S, D, T)
+    # the kernel moves 16-byte pieces of K and 4-byte pieces of V
+    if k.data_ptr() % 16:
+        k = k.clone()
+    if payload.data_ptr() % 4:
+        payload = payload.clone()
+    nb = -(-T // BLOCK)
+    pages = B * nb
+    k_bytes, v_bytes, s_bytes = pages * KV * BLOCK * D * 2, pages * KV * BLOCK * D, pages * KV * BLOCK * 4
+    buf = torch.empty(k_bytes + v_bytes + s_bytes + pages * 4, dtype=torch.uint8, device=dev)
+    kp = buf.data_ptr()
+    vp = kp + k_bytes
+    sp = vp + v_bytes
+    bt = sp + s_bytes
+    st = _stream(dev)
+    _native.check(lib.sdv_pack_contiguous(_p(k), _p(payload), _p(scale), B, KV, T, D, kp, vp, sp, bt, st),
+                  "sdv_pack_contiguous")
+    out = torch.empty_like(q)
+    ws = workspace(dev, nbytes)
+    _native.check(lib.sdv_paged_attention(_p(q), kp, vp, sp, pages, 0, 0, 0, bt, nb, None, 1, B, H, KV, S, D, T, 0,
+                                          _p(ws), ws.numel(), _p(out), st), "sdv_paged_attention")
+    if _CHECK_SYNC:
+        check_workspace(ws)
+    return out
 
 
 def fp8_encode(x: torch.Tensor) -> torch.Tensor:
@@ -455,6 +498,16 @@ def _lib_paged_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.
 
 @_lib_paged_attention.register_fake
 def _(q, k_pages, v_pages, v_scales, block_table, seq_lens, max_seq_len, q_token_major=False):
+    return torch.empty_like(q)
+
+
+@torch.library.custom_op("sdv::attention", mutates_args=())
+def _lib_attention(q: torch.Tensor, k: torch.Tensor, v_payload: torch.Tensor, v_scale: torch.Tensor) -> torch.Tensor:
+    return _contiguous_attention(q, k, v_payload, v_scale)
+
+
+@_lib_attention.register_fake
+def _(q, k, v_payload, v_scale):
     return torch.empty_like(q)
 
 
