@@ -105,6 +105,18 @@ int sdv_quant_append_tiles(const void* v_new, const void* k_new, const int32_t* 
                            int64_t k_layer_stride, int64_t v_layer_stride, int64_t s_layer_stride,
                            int32_t scale_mode, const int32_t* tile_starts, int32_t n_tiles, void* stream);
 
+/*
+ * Slot mapping and tile table of whole prompts packed back to back, for sdv_quant_append_tiles:
+ * lengths is a HOST array [batch], sequence b's rows follow those of the sequences before it, its
+ * first token at position 0.  slots int32 [sum(lengths)]: the block-table slot of each row;
+ * tile_starts int32 [sum(ceil(lengths/16)) + 1] or NULL: a tile per page block, the last entry the
+ * row count.  Each length is at most 16 * max_blocks_per_seq and its block ids are valid (they are
+ * not checked).  The lengths travel as kernel arguments: nothing is copied from the host.  No
+ * counterpart in the reference.
+ */
+int sdv_varlen_slots(const int32_t* block_table, int32_t max_blocks_per_seq, const int32_t* lengths,
+                     int32_t batch, int32_t* slots, int32_t* tile_starts, void* stream);
+
 /* Bytes of workspace sdv_paged_attention needs for these sizes (0 on invalid sizes). */
 size_t sdv_attention_workspace_size(int32_t num_layers, int32_t batch, int32_t q_heads,
                                     int32_t kv_heads, int32_t q_len, int32_t head_dim,

@@ -212,9 +212,80 @@ __global__ __launch_bounds__(64 * kQuantWaves) void quant_append_kernel(QuantArg
   }
 }
 
+// ---------------------------------------------------------------------------- varlen slots
+// Slots and tile starts of whole prompts packed back to back (sequence b's rows begin where those
+// before it end, its first token at position 0), from the block table on the device: a thread per
+// row finds its sequence among the starts, which travel as kernel arguments, so nothing is copied
+// from the host.  Latency-bound (16K rows 3.4 us); the same arrays built on the host and copied took
+// 290 us (slots) and 123 us (tiles) for 8 prompts of 100 to 4000 tokens.
+constexpr int kVarlenSeqs = 256;  // sequences per launch
+
+struct VarlenArgs {
+  const int32_t* block_table;
+  int32_t* slots;
+  int32_t* tiles;  // nullptr: slots only
+  int max_blocks, n_seqs;
+  int rows[kVarlenSeqs + 1];    // first row of each sequence, and the end of the last
+  int tile0[kVarlenSeqs + 1];   // first tile of each, and the end
+};
+
+__global__ __launch_bounds__(256) void varlen_slots_kernel(VarlenArgs a) {
+  const int row = a.rows[0] + (int)(blockIdx.x * 256 + threadIdx.x);
+  if (row >= a.rows[a.n_seqs]) return;
+  int lo = 0, hi = a.n_seqs;  // rows[lo] <= row < rows[hi]: of equal starts (empty sequences) the last
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (a.rows[mid] <= row)
+      lo = mid;
+    else
+      hi = mid;
+  }
+  const int pos = row - a.rows[lo];
+  a.slots[row] = a.block_table[(int64_t)lo * a.max_blocks + (pos >> 4)] * kBlock + (pos & (kBlock - 1));
+  if (a.tiles) {
+    if ((pos & (kBlock - 1)) == 0) a.tiles[a.tile0[lo] + (pos >> 4)] = row;
+    if (row == a.rows[a.n_seqs] - 1) a.tiles[a.tile0[a.n_seqs]] = row + 1;  // the table's end, or the next launch's start
+  }
+}
+
 }  // namespace sdv
 
 using namespace sdv;
+
+extern "C" int sdv_varlen_slots(const int32_t* block_table, int32_t max_blocks_per_seq, const int32_t* lengths,
+                                int32_t batch, int32_t* slots, int32_t* tile_starts, void* stream) {
+  if (!block_table || !lengths || !slots) return SDV_ERR_NULL;
+  if (batch <= 0 || max_blocks_per_seq <= 0) return SDV_ERR_SHAPE;
+  int64_t total = 0;
+  for (int b = 0; b < batch; ++b) {
+    if (lengths[b] < 0 || lengths[b] > (int64_t)max_blocks_per_seq * kBlock) return SDV_ERR_SHAPE;
+    total += lengths[b];
+  }
+  if (total > INT32_MAX - 256) return SDV_ERR_SHAPE;
+  if (!aligned(block_table, 4) || !aligned(slots, 4) || !aligned(tile_starts, 4)) return SDV_ERR_ALIGN;
+  if (total == 0) return SDV_OK;  // no rows: the caller's tables are empty
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  int row = 0, tile = 0;
+  for (int b0 = 0; b0 < batch; b0 += kVarlenSeqs) {
+    VarlenArgs a;
+    a.block_table = block_table + (int64_t)b0 * max_blocks_per_seq;
+    a.slots = slots;
+    a.tiles = tile_starts;
+    a.max_blocks = max_blocks_per_seq;
+    a.n_seqs = batch - b0 < kVarlenSeqs ? batch - b0 : kVarlenSeqs;
+    for (int i = 0; i < a.n_seqs; ++i) {
+      a.rows[i] = row;
+      a.tile0[i] = tile;
+      row += lengths[b0 + i];
+      tile += (lengths[b0 + i] + kBlock - 1) / kBlock;
+    }
+    a.rows[a.n_seqs] = row;
+    a.tile0[a.n_seqs] = tile;
+    const int n = row - a.rows[0];
+    if (n > 0) hipLaunchKernelGGL(varlen_slots_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a);
+  }
+  return hipGetLastError() == hipSuccess ? SDV_OK : SDV_ERR_HIP;
+}
 
 static int quant_append(const void* v_new, const void* k_new, const int32_t* slot_mapping, int32_t n_tokens,
                         int32_t kv_heads, int32_t head_dim, int32_t group_size, int32_t num_layers,

@@ -48,6 +48,7 @@ SIGNATURES = {
                                         _P, _P, _P, _I32, _I64, _I64, _I64, _I32, _P]),
     "sdv_quant_append_tiles": (ctypes.c_int, [_P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I64,
                                               _P, _P, _P, _I32, _I64, _I64, _I64, _I32, _P, _I32, _P]),
+    "sdv_varlen_slots": (ctypes.c_int, [_P, _I32, ctypes.POINTER(_I32), _I32, _P, _P, _P]),
     "sdv_attention_workspace_size": (_SZ, [_I32, _I32, _I32, _I32, _I32, _I32, _I32]),
     "sdv_attention_workspace_init": (ctypes.c_int, [_P, _SZ, _P]),
     "sdv_attention_workspace_status": (ctypes.c_int, [_P, _SZ, ctypes.POINTER(ctypes.c_uint32),

@@ -97,7 +97,7 @@ class PagedKVCache:
         self.blocks: list[list[int]] = [[] for _ in range(batch)]
         self.lengths: list[int] = [0] * batch
         self._bt = None
-        self._tiles = None  # (lengths, device tile table) of the last prefill
+        self._tiles = None  # (lengths, stream, device tile table) of the last prefill
         self._ws = None     # attention workspace owned by the pool
         # replaced workspaces, kept alive for graphs that recorded them; each replacement is at
         # least twice the size of the one before, so they hold at most the current one's bytes
@@ -247,7 +247,10 @@ class PagedKVCache:
                                    scale_mode=self.scale_mode)
 
     def varlen_slots(self, lengths: list[int]) -> torch.Tensor:
-        """int32 (sum(lengths),) slots of positions 0..lengths[b]-1 of each sequence in turn."""
+        """int32 (sum(lengths),) slots of positions 0..lengths[b]-1 of each sequence in turn (on a
+        device, written by a kernel on the current stream)."""
+        if self.device.type == "cuda" and not _recording(self.device):
+            return self._varlen(lengths, tiles=False)[0]
         out = []
         for b, n in enumerate(lengths):
             pos = torch.arange(n, dtype=torch.int64)
@@ -255,28 +258,44 @@ class PagedKVCache:
             out.append(blk[pos // BLOCK] * BLOCK + pos % BLOCK)
         return torch.cat(out).to(torch.int32).to(self.device)
 
+    def _varlen(self, lengths: list[int], tiles: bool = True):
+        """(slots, tile table or None) of whole prompts: the device's block table expanded by one
+        kernel, the lengths as its arguments."""
+        for b, n in enumerate(lengths):
+            if n < 0 or -(-n // BLOCK) > len(self.blocks[b]):
+                raise IndexError(f"sequence {b} has {len(self.blocks[b])} blocks, {n} positions asked for")
+        return ops.varlen_slots(self.block_table(), lengths, tiles=tiles)
+
     def prefill(self, layer: int, k_new: torch.Tensor, v_new: torch.Tensor, lengths: list[int],
                 slots: torch.Tensor | None = None) -> torch.Tensor:
         """Write whole prompts of different lengths into one layer (one kernel 1 launch).
 
         k_new/v_new BF16 (sum(lengths), KV, D), sequence after sequence (the varlen layout);
-        lengths become ``lengths``.  Returns the slot mapping so that later layers can pass it.
-        The launch takes a tile table that starts a tile at every sequence's first row (built
-        once per set of lengths), so whole page blocks are written with 16-byte stores.
+        lengths become ``lengths``.  Returns the slot mapping so that later layers can pass it
+        (written by a kernel on the current stream, like any result).  The launch takes a tile
+        table that starts a tile at every sequence's first row (built with the slots, once per set
+        of lengths and stream), so whole page blocks are written with 16-byte stores.
         """
         if len(lengths) != self.batch:
             raise ValueError(f"{len(lengths)} lengths for a batch of {self.batch}")
         for b, n in enumerate(lengths):
             self.reserve(b, n)
-        if slots is None:
-            slots = self.varlen_slots(lengths)
-        key = tuple(lengths)
-        if self._tiles is None or self._tiles[0] != key:
-            t = torch.tensor(ops.varlen_tile_starts(list(lengths)), dtype=torch.int32).to(self.device)
-            self._tiles = (key, t)
+        on_device = self.device.type == "cuda"
+        key = (tuple(lengths), ops._stream(self.device) if on_device else 0)
+        stale = self._tiles is None or self._tiles[:2] != key
+        if on_device and (slots is None or stale) and not _recording(self.device):
+            fresh, table = self._varlen(lengths)
+            slots = fresh if slots is None else slots
+            self._tiles = (*key, table)
+        else:
+            if slots is None:
+                slots = self.varlen_slots(lengths)
+            if stale:
+                table = torch.tensor(ops.varlen_tile_starts(list(lengths)), dtype=torch.int32).to(self.device)
+                self._tiles = (*key, table)
         kp, vp, vs = self.layer(layer)
         ops.quant_append(v_new, slots, kp, vp, vs, k_new, scale_mode=self.scale_mode,
-                         tile_starts=self._tiles[1])
+                         tile_starts=self._tiles[2])
         for b, n in enumerate(lengths):
             self.lengths[b] = n
         return slots

@@ -267,6 +267,24 @@ def quant_append(v_new: torch.Tensor, slot_mapping: torch.Tensor, k_pages: torch
     _native.check(st, "sdv_quant_append_tiles")
 
 
+def varlen_slots(block_table: torch.Tensor, lengths: list[int], tiles: bool = True):
+    """(slots, tile_starts) of whole prompts packed back to back: the slot of every row, from the
+    block table int32 (B, max_blocks), and varlen_tile_starts(lengths) as a tensor (None without
+    ``tiles``), in one kernel on the current stream (sdv_varlen_slots)."""
+    _need(block_table, "block_table", (torch.int32,), ndim=(2,))
+    n = len(lengths)
+    if n > block_table.shape[0]:
+        _fail(f"{n} lengths for a block table of {block_table.shape[0]} sequences")
+    dev = block_table.device
+    slots = torch.empty(sum(lengths), dtype=torch.int32, device=dev)
+    table = torch.empty(sum(-(-x // BLOCK) for x in lengths) + 1, dtype=torch.int32, device=dev) if tiles else None
+    if slots.numel() == 0:
+        return slots, table.zero_() if tiles else None
+    _native.check(_native.load().sdv_varlen_slots(_p(block_table), block_table.shape[1], (ctypes.c_int32 * n)(*lengths), n,
+                                                  _p(slots), _p(table), _stream(dev)), "sdv_varlen_slots")
+    return slots, table
+
+
 def varlen_tile_starts(lengths: list[int], starts: list[int] | None = None) -> list[int]:
     """Tile table for a packed varlen input of sequences with `lengths` tokens whose first token
     lands at position `starts[b]` of its sequence (0: a whole prompt): tiles break where a page

@@ -19,3 +19,17 @@ def test_host_validation():
     assert f(k=ctypes.c_void_p(0x1008)) == _native.SDV_ERR_ALIGN
     assert f(kp=ctypes.c_void_p(0x1008)) == _native.SDV_ERR_ALIGN
     assert f(v=ctypes.c_void_p(0x1002)) == _native.SDV_ERR_ALIGN
+
+
+def test_varlen_slots_host_validation():
+    lib = _native.load()
+
+    def f(bt=P, mb=4, lens=(5, 64), slots=P, tiles=P, n=None):
+        arr = (ctypes.c_int32 * max(1, len(lens)))(*lens) if lens is not None else None
+        return lib.sdv_varlen_slots(bt, mb, arr, len(lens) if n is None else n, slots, tiles, None)
+    assert f(bt=None) == _native.SDV_ERR_NULL and f(slots=None) == _native.SDV_ERR_NULL
+    assert f(lens=None, n=2) == _native.SDV_ERR_NULL
+    assert f(lens=(5, 65)) == _native.SDV_ERR_SHAPE and f(lens=(-1,)) == _native.SDV_ERR_SHAPE
+    assert f(n=0) == _native.SDV_ERR_SHAPE and f(mb=0) == _native.SDV_ERR_SHAPE
+    assert f(tiles=ctypes.c_void_p(0x1002)) == _native.SDV_ERR_ALIGN
+    assert f(lens=(0, 0)) == _native.SDV_OK      # no rows: nothing to do, no launch
