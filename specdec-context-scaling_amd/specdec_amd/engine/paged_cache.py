@@ -123,6 +123,22 @@ class PagedKVCache:
         self.k_pages, self.v_pages, self.v_scales = k, v, s
         self.alloc.grow(new)
 
+    def _layer_pointers(self, i: int, device: torch.device):
+        """(K, V, scale addresses of layer i, blocks), or None where the page tensors are not what
+        _new_pages made or not on `device` (the general path then says what is wrong)."""
+        k, v, s = self.k_pages, self.v_pages, self.v_scales
+        L, KV, D = self.num_layers, self.kv_heads, self.head_dim
+        shape = k.shape
+        if not 0 <= i < L or len(shape) != 6 or k.device != device or v.device != device or s.device != device:
+            return None
+        nb = shape[1]
+        if shape != (L, nb, KV, D // 8, BLOCK, 8) or v.shape != (L, nb, KV, D, BLOCK) or s.shape != (L, nb, KV, BLOCK) or \
+                k.dtype is not torch.bfloat16 or v.dtype is not torch.uint8 or s.dtype is not torch.float32 or \
+                not (k.is_contiguous() and v.is_contiguous() and s.is_contiguous()):
+            return None
+        n = i * nb * KV * BLOCK  # scales per layer
+        return k.data_ptr() + n * D * 2, v.data_ptr() + n * D, s.data_ptr() + n * 4, nb
+
     def layer(self, i: int):
         """(k_pages, v_pages, v_scales) of layer i (contiguous views)."""
         return self.k_pages[i], self.v_pages[i], self.v_scales[i]
@@ -234,13 +250,21 @@ class PagedKVCache:
             self.reserve(b, starts[b] + S)
         for b in range(B):
             self.lengths[b] = starts[b] + S
-        kp, vp, vs = self.layer(layer)
-        shp = (B * S, self.kv_heads, self.head_dim)
         tmax = max(self.lengths)
         uniform = all(n == tmax for n in self.lengths)
         H = q.shape[2] if q_token_major else q.shape[1]
         self._q_heads, self._q_len = max(self._q_heads, H), max(self._q_len, S)
         ws = self.workspace(ops.attention_workspace_bytes(1, B, H, self.kv_heads, S, self.head_dim, tmax))
+        if uniform and out is None:
+            # the engine's per-layer call: its host cost is part of every token, so what the
+            # general path checks one helper call at a time is tested here in one expression, and
+            # anything unusual goes there
+            got = ops.append_attend_pages(q, k_new, v_new, self._layer_pointers(layer, q.device), self.block_table(), tmax,
+                                          B, S, H, self.kv_heads, self.head_dim, bool(q_token_major), ws, self.scale_mode)
+            if got is not None:
+                return got
+        kp, vp, vs = self.layer(layer)
+        shp = (B * S, self.kv_heads, self.head_dim)
         return ops.paged_attention(q, kp, vp, vs, self.block_table(), None if uniform else self.seq_lens_tensor(),
                                    tmax, q_token_major=q_token_major, out=out, workspace_tensor=ws,
                                    append=(k_new.reshape(shp), v_new.reshape(shp), None),
@@ -279,7 +303,8 @@ class PagedKVCache:
         if len(lengths) != self.batch:
             raise ValueError(f"{len(lengths)} lengths for a batch of {self.batch}")
         for b, n in enumerate(lengths):
-            self.reserve(b, n)
+            if n > len(self.blocks[b]) * BLOCK:
+                self.reserve(b, n)
         on_device = self.device.type == "cuda"
         key = (tuple(lengths), ops._stream(self.device) if on_device else 0)
         stale = self._tiles is None or self._tiles[:2] != key
@@ -293,11 +318,12 @@ class PagedKVCache:
             if stale:
                 table = torch.tensor(ops.varlen_tile_starts(list(lengths)), dtype=torch.int32).to(self.device)
                 self._tiles = (*key, table)
-        kp, vp, vs = self.layer(layer)
-        ops.quant_append(v_new, slots, kp, vp, vs, k_new, scale_mode=self.scale_mode,
-                         tile_starts=self._tiles[2])
-        for b, n in enumerate(lengths):
-            self.lengths[b] = n
+        pages = self._layer_pointers(layer, v_new.device) if on_device else None
+        if not ops.quant_append_pages(v_new, k_new, slots, pages, self._tiles[2], self.kv_heads, self.head_dim, self.scale_mode):
+            kp, vp, vs = self.layer(layer)
+            ops.quant_append(v_new, slots, kp, vp, vs, k_new, scale_mode=self.scale_mode,
+                             tile_starts=self._tiles[2])
+        self.lengths[:] = lengths
         return slots
 
     def seq_lens_tensor(self, lengths: list[int] | None = None) -> torch.Tensor:

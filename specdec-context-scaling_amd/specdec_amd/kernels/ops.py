@@ -96,6 +96,30 @@ def _pages_dims(k_pages, v_pages, v_scales, layered: bool):
     return nb, kv, d
 
 
+def _plain_pages(q, k_pages, v_pages, v_scales, block_table, seq_lens):
+    """(blocks, KV heads, head_dim) when every tensor of a paged_attention call is what _need and
+    _pages_dims ask for, tested in one pass (the engine calls it per layer and token); else None."""
+    try:
+        dev, ks = q.device, k_pages.shape
+        lead = len(q.shape) - 4
+        if lead not in (0, 1) or len(ks) != 5 + lead:
+            return None
+        nb, kv, dc, blk, eight = ks[lead:]
+        front = ks[:lead + 2]
+        if (blk == BLOCK and eight == 8 and v_pages.shape == (*front, dc * 8, BLOCK) and v_scales.shape == (*front, BLOCK)
+                and q.is_cuda and k_pages.device == dev and v_pages.device == dev and v_scales.device == dev
+                and block_table.device == dev and q.dtype is torch.bfloat16 and k_pages.dtype is torch.bfloat16
+                and v_pages.dtype is torch.uint8 and v_scales.dtype is torch.float32 and block_table.dtype is torch.int32
+                and len(block_table.shape) == 2 and q.is_contiguous() and k_pages.is_contiguous() and v_pages.is_contiguous()
+                and v_scales.is_contiguous() and block_table.is_contiguous()
+                and (seq_lens is None or (seq_lens.device == dev and seq_lens.dtype is torch.int32
+                                          and len(seq_lens.shape) == 1 and seq_lens.is_contiguous()))):
+            return nb, kv, dc * 8
+    except AttributeError:  # not a tensor
+        pass
+    return None
+
+
 def new_workspace(device: torch.device, nbytes: int) -> torch.Tensor:
     """A fresh uint8 workspace of at least nbytes whose synchronisation prefix is zeroed
     (sdv_attention_workspace_init on the current stream)."""
@@ -328,16 +352,20 @@ def paged_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tenso
     table on the device.
     """
     lib = _native.load()
-    _need(q, "q", (torch.bfloat16,), ndim=(4, 5))
+    dims = _plain_pages(q, k_pages, v_pages, v_scales, block_table, seq_lens)
+    if dims is None:  # something unusual, or wrong: one check at a time says what
+        _need(q, "q", (torch.bfloat16,), ndim=(4, 5))
+        dev = q.device
+        _need(k_pages, "k_pages", (torch.bfloat16,), dev)
+        _need(v_pages, "v_pages", (torch.uint8, torch.float8_e4m3fn), dev)
+        _need(v_scales, "v_scales", (torch.float32,), dev)
+        _need(block_table, "block_table", (torch.int32,), dev, ndim=(2,))
+        if seq_lens is not None:
+            _need(seq_lens, "seq_lens", (torch.int32,), dev, ndim=(1,))
+        dims = _pages_dims(k_pages, v_pages, v_scales, q.dim() == 5)
+    nb, kv, d = dims
     dev = q.device
     layered = q.dim() == 5
-    _need(k_pages, "k_pages", (torch.bfloat16,), dev)
-    _need(v_pages, "v_pages", (torch.uint8, torch.float8_e4m3fn), dev)
-    _need(v_scales, "v_scales", (torch.float32,), dev)
-    _need(block_table, "block_table", (torch.int32,), dev, ndim=(2,))
-    if seq_lens is not None:
-        _need(seq_lens, "seq_lens", (torch.int32,), dev, ndim=(1,))
-    nb, kv, d = _pages_dims(k_pages, v_pages, v_scales, layered)
     L = q.shape[0] if layered else 1
     if layered and k_pages.shape[0] != L:
         _fail(f"q has {L} layers, pages have {k_pages.shape[0]}")
@@ -369,8 +397,9 @@ def paged_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tenso
         ref = _READY.get(id(workspace_tensor))
         if ref is None or ref() is not workspace_tensor:  # a caller's own buffer: zero its sync prefix once
             _init_workspace(workspace_tensor)
-    per = lambda t: t[0].numel() if layered else 0  # noqa: E731
-    args = (_p(q), _p(k_pages), _p(v_pages), _p(v_scales), nb, per(k_pages), per(v_pages), per(v_scales),
+    per = lambda t: t[0].numel()  # noqa: E731
+    k_ls, v_ls, s_ls = (per(k_pages), per(v_pages), per(v_scales)) if layered else (0, 0, 0)
+    args = (_p(q), _p(k_pages), _p(v_pages), _p(v_scales), nb, k_ls, v_ls, s_ls,
             _p(block_table), block_table.shape[1], _p(seq_lens), L, B, H, kv, S, d, max_seq_len,
             int(bool(q_token_major)), _p(workspace_tensor), workspace_tensor.numel(), _p(out), _stream(dev))
     if append is not None:
@@ -392,7 +421,7 @@ def paged_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tenso
             k_new = k_new.clone()
         if v_new.data_ptr() % 16:
             v_new = v_new.clone()
-        st = lib.sdv_paged_attention_append(*args[:-1], _p(k_new), _p(v_new), _p(slots), per(v_new),
+        st = lib.sdv_paged_attention_append(*args[:-1], _p(k_new), _p(v_new), _p(slots), per(v_new) if layered else 0,
                                             _SCALE_MODES[scale_mode], args[-1])
         _native.check(st, "sdv_paged_attention_append")
         if _CHECK_SYNC:
@@ -406,6 +435,55 @@ def paged_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tenso
     if _CHECK_SYNC:
         check_workspace(workspace_tensor)
     return out
+
+
+def _plain(t, dtype, dev, shape) -> bool:
+    """A contiguous device tensor of this type and shape whose first byte is 16-byte aligned."""
+    return (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is dtype and t.device == dev and t.shape == shape
+            and t.is_contiguous() and t.data_ptr() % 16 == 0)
+
+
+def append_attend_pages(q, k_new, v_new, pages, block_table, max_seq_len, B, S, H, KV, D, token_major, ws, scale_mode):
+    """paged_attention(..., append=(k_new, v_new, None)) of one layer of a pool whose page
+    addresses the caller has (`pages`: K, V, scales, blocks), every sequence max_seq_len tokens
+    long; k_new/v_new (B, S, KV, D).  None when an argument is not the plain tensor that the fixed
+    arguments of the call stand for: paged_attention then takes it, or says what is wrong."""
+    dev = q.device
+    if pages is None or scale_mode not in _SCALE_MODES or H % KV or \
+            not _plain(q, torch.bfloat16, dev, (B, S, H, D) if token_major else (B, H, S, D)) or \
+            not _plain(k_new, torch.bfloat16, dev, (B, S, KV, D)) or not _plain(v_new, torch.bfloat16, dev, (B, S, KV, D)) or \
+            not (block_table.device == dev and block_table.dtype is torch.int32 and block_table.is_contiguous()) or \
+            block_table.shape[0] != B or max_seq_len <= 0 or block_table.shape[1] * BLOCK < max_seq_len or ws.device != dev:
+        return None
+    out = torch.empty_like(q)
+    kp, vp, sp, nb = pages
+    st = _native.load().sdv_paged_attention_append(
+        q.data_ptr(), kp, vp, sp, nb, 0, 0, 0, block_table.data_ptr(), block_table.shape[1], None, 1, B, H, KV, S, D,
+        max_seq_len, int(token_major), ws.data_ptr(), ws.numel(), out.data_ptr(), k_new.data_ptr(), v_new.data_ptr(), None, 0,
+        _SCALE_MODES[scale_mode], _stream(dev))
+    if st:
+        _native.check(st, "sdv_paged_attention_append")
+    if _CHECK_SYNC:
+        check_workspace(ws)
+    return out
+
+
+def quant_append_pages(v_new, k_new, slots, pages, tile_starts, KV, D, scale_mode) -> bool:
+    """quant_append of one layer of a pool whose page addresses the caller has; False (nothing
+    done) when an argument is not the plain tensor that the call's fixed arguments stand for."""
+    if pages is None or not isinstance(v_new, torch.Tensor) or v_new.dim() != 3 or scale_mode not in _SCALE_MODES:
+        return False
+    dev, n = v_new.device, v_new.shape[0]
+    if not _plain(v_new, torch.bfloat16, dev, (n, KV, D)) or not _plain(k_new, torch.bfloat16, dev, (n, KV, D)) or \
+            not _plain(slots, torch.int32, dev, (n,)) or tile_starts.device != dev:
+        return False
+    kp, vp, sp, nb = pages
+    st = _native.load().sdv_quant_append_tiles(
+        v_new.data_ptr(), k_new.data_ptr(), slots.data_ptr(), n, KV, D, D, 1, 0, kp, vp, sp, nb, 0, 0, 0,
+        _SCALE_MODES[scale_mode], tile_starts.data_ptr(), tile_starts.shape[0] - 1, _stream(dev))
+    if st:
+        _native.check(st, "sdv_quant_append_tiles")
+    return True
 
 
 def pack_contiguous(k: torch.Tensor, v_payload: torch.Tensor, v_scale: torch.Tensor):

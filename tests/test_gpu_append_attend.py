@@ -156,3 +156,45 @@ def test_append_attend_rejects_bad_shapes(cuda_device):
     slots = torch.zeros((1,), dtype=torch.int32, device=cuda_device)
     with pytest.raises(Exception):
         ops.paged_attention(q, kp, vp, vs, bt, sl, 16, append=(kn, kn, slots))
+
+
+def test_pool_calls_take_unusual_tensors(cuda_device):
+    """append_attend and prefill test the plain case in one expression; misaligned,
+    strided and wrong arguments go the general way: the same pages and output, the same refusals."""
+    announce("append_attend and prefill with unusual tensors")
+    g = wl.gen(77, cuda_device)
+    h, kv, d, t0, s = 12, 2, 128, 40, 3
+    k = torch.randn((1, t0 + s, kv, d), generator=g, device=cuda_device).to(torch.bfloat16)
+    q = torch.randn((1, s, h, d), generator=g, device=cuda_device).to(torch.bfloat16)
+
+    def off(x):       # the same values from a buffer that starts off a 16-byte boundary
+        buf = torch.empty(x.numel() + 1, dtype=x.dtype, device=x.device)
+        buf[1:] = x.flatten()
+        return buf[1:].view(x.shape)
+
+    def strided(x):   # as a transposed view
+        return x.transpose(1, 2).contiguous().transpose(1, 2)
+
+    got = []
+    for f in (lambda x: x, off):
+        cache = PagedKVCache(kv, d, num_layers=2, num_blocks=4, device=cuda_device, seed=8)
+        first = off(k[0, :t0]) if f is off else k[0, :t0]
+        cache.prefill(1, first, first, [t0])
+        out = cache.append_attend(1, q, f(k[:, t0:]), f(k[:, t0:]), q_token_major=True)
+        got.append((out, cache.k_pages.clone(), cache.v_pages.clone(), cache.v_scales.clone()))
+        again = cache.append_attend(-1, q, f(k[:, t0:]), f(k[:, t0:]), [t0], q_token_major=True)   # layer from the end
+        assert torch.equal(again, out)
+    for other in got[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(got[0], other))
+    new = k[:, t0:]
+    for bad in (dict(q=q.float()), dict(q=q[..., :64].contiguous()), dict(k=new.float()), dict(v=new[..., :64].contiguous()),
+                dict(q=q.transpose(2, 3)), dict(k=new.cpu()), dict(v=strided(new))):
+        with pytest.raises(RuntimeError):
+            cache.append_attend(0, bad.get("q", q), bad.get("k", new), bad.get("v", new), [t0], q_token_major=True)
+    with pytest.raises(IndexError):
+        cache.append_attend(2, q, new, new, [t0], q_token_major=True)
+    for x in (k[0].float(), strided(k)[0]):
+        with pytest.raises(RuntimeError):
+            cache.prefill(0, x, x, [t0 + s])
+    with pytest.raises(RuntimeError):
+        cache.prefill(0, k[0], k[0], [t0])
