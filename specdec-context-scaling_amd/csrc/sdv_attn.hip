@@ -2063,18 +2063,18 @@ static void plan_prefill(int64_t groups, int R, int S, int G, int D, int T, Plan
   const int64_t slot_b = (int64_t)kPfRows * D * 4;
   p->pf_slots = (int)(slots / slot_b);
   const int64_t have = p->pf_slots + (int64_t)(kSyncPartBytes - kPfDescBytes) / slot_b;
-  const int64_t cap1 = kPfCus * pf_wgs_per_cu(D, false), cap2 = kPfCus * pf_wgs_per_cu(D, true);
+  const int64_t cap = kPfWorkgroups;
   p->pf_min1 = p->pf_min2 = kPfMinStages;
   // A range's partial row groups need a slot each: W + nrg in all, and 2 per workgroup at most
-  const int64_t w2 = std::min({cap2, std::max(have / 2, have - nrg), (U + kPfMinStages - 1) / kPfMinStages});
-  if (U >= (1 << 30) || nbk >= (1 << 22) || nrg > kPfMaxGroups || w2 < std::min(nrg, cap2)) return;  // whole row groups
+  const int64_t w2 = std::min({cap, std::max(have / 2, have - nrg), (U + kPfMinStages - 1) / kPfMinStages});
+  if (U >= (1 << 30) || nbk >= (1 << 22) || nrg > kPfMaxGroups || w2 < std::min(nrg, cap)) return;  // whole row groups
   p->pf_w2 = (int)w2;
   p->pf_dense = w2 + nrg <= have;
   // pass 1: the ranges that cut a row group of ns stages, at most (ns - 2) / per + 2, fit its
   // statistics
   const int ns = pf_stages(p->pf_nrg - 1, S, G, T);
   if (p->pf_split >= 2) {
-    p->pf_w1 = (int)std::min(cap1, (U + kPfMinStages - 1) / kPfMinStages);
+    p->pf_w1 = (int)std::min(cap, (U + kPfMinStages - 1) / kPfMinStages);
     p->pf_min1 = std::max(p->pf_min1, (ns - 1 + p->pf_split - 2) / (p->pf_split - 1));
   }
 }

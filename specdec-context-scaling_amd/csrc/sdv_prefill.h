@@ -34,7 +34,7 @@
 // (head_dim 128; MFMA 2,048).  Measured, both passes, of one KV pair's 2048 rows x 8192 keys
 // (12/2/128, 14/2/64), 777 x 5000 (14/2/64), 2048 x 2048 and 300 x 5000 (12/2/128), before (16x16
 // MFMAs, a row group's rows of one head, parts per row group) and now:
-//   233 -> 184, 152 -> 123, 83 -> 58, 77 -> 73, 74 -> 62 us.
+//   233 -> 183, 152 -> 122, 83 -> 56, 77 -> 61, 74 -> 54 us.
 // What it took: one wave's LDS operand reads run across the stage barrier (three buffers, waits
 // counted by hand: 92 -> 80 us of pass 2's loop), the parts' sum in its own launch (the last part
 // to finish summing 470 KB alone held the end up by 29 us), q.k^T, scores and p.V of three units
@@ -49,12 +49,16 @@ constexpr int kPfStage = 64;                   // keys per stage: two units of 3
 constexpr int kPfIds = 2048;                   // page ids staged in LDS at a time (a multiple of 4)
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// Workgroups of 8 wavefronts a CU holds: pass 1 and head_dim 64 two, pass 2 for head_dim 128 one
-// (64 accumulators per lane).
-constexpr int pf_wgs_per_cu(int D, bool OUT) { return OUT ? 1 : 2; }
-constexpr int kPfCus = 256;
-constexpr int kPfMinStages = 4;                // fewest stages of a workgroup's range
-constexpr int kPfSegStages = 2;                // stages that starting a row group costs, about
+// One workgroup per CU, two wavefronts per SIMD: pass 2 for head_dim 128 needs the registers (64
+// accumulators per lane), and with two workgroups per CU the others were no faster over long
+// ranges (pass 1 of 2048 x 8192 76 us either way) and paid twice the starts (2048 x 2048 28.9
+// against 22.2 us).
+constexpr int kPfWorkgroups = 256;
+// Fewest stages of a workgroup's range (150 x 400 of 14/2/64: 30 us with 6, 27 with 4, 24.7 with 3)
+constexpr int kPfMinStages = 3;
+// Stages that starting a row group costs, about (777 x 5000 of 14/2/64: 61 us with 2, 58 with 4, 56
+// with 6; 100 x 16000 of 12/2/128 76, 75, 68)
+constexpr int kPfSegStages = 6;
 
 // Stages of row group i (of S tokens x G heads) over T keys; at least one, so that a row group
 // that sees nothing still has a workgroup to write its zeros.
@@ -103,7 +107,7 @@ __device__ __forceinline__ float4* pf_slot(const AttnArgs& a, int D, int w0, int
 }
 
 template <int D, bool OUT>
-__global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(2 * pf_wgs_per_cu(D, OUT))))
+__global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_kernel(AttnArgs a, int layers) {
   constexpr int W = kPfWaves, NTHR = 64 * W;
   constexpr int KS = D / 16;        // MFMA steps of one q.k^T product over the head dimension
@@ -121,6 +125,8 @@ void prefill_kernel(AttnArgs a, int layers) {
   // a row group's weight in the order: its stages and, before them, the cost of its start
   auto weight_of = [&](int f) { return kPfSegStages + pf_stages(f % nrg, a.S, a.G, seq_len_of(a, f / nrg)); };
 
+  int window = 0;  // page-id windows staged so far
+  if (tid == 0) s_bad = 0;
   // ---- this workgroup's range of stages
   PfPos pos;
   int u = 0, uend = 0;       // current stage and end of the range
@@ -134,26 +140,28 @@ void prefill_kernel(AttnArgs a, int layers) {
     u = 0;
     uend = pos.wt;
   } else {
-    // stages of the row groups of one (layer, KV head), scanned NTHR at a time: `lo` of this
-    // thread's row group, and the sum C of all
-    int v = tid < nf ? weight_of(tid) : 0, inc = wave_scan(v);
-    if (lane == 63) s_scan[wave] = inc;
-    int rest = 0;
-    for (int f = NTHR + tid; f < nf; f += NTHR) rest += weight_of(f);
-    if (nf > NTHR) {  // workgroup-uniform
+    // weights of the row groups of one (layer, KV head): each wavefront scans up to 64 of them in
+    // its lanes, more are scanned NTHR at a time by the workgroup; `lo` of this thread's row
+    // group, `first` of those scanned so far, and the sum C of all
+    const bool few = nf <= kWave;
+    const int f0 = few ? lane : tid;
+    int v = f0 < nf ? weight_of(f0) : 0, inc = wave_scan(v);
+    int lo = inc - v, first = __builtin_amdgcn_readlane(inc, 63), C = first;
+    if (!few) {  // workgroup-uniform
+      if (lane == 63) s_scan[wave] = inc;
+      int rest = 0;
+      for (int f = NTHR + tid; f < nf; f += NTHR) rest += weight_of(f);
       rest = wave_scan(rest);
       if (lane == 63) s_rest[wave] = rest;
-    }
-    __syncthreads();
-    int lo = inc - v, first = 0, C = 0;
+      __syncthreads();
+      first = C = 0;
 #pragma unroll
-    for (int i = 0; i < W; ++i) {
-      lo += i < wave ? s_scan[i] : 0;
-      first += s_scan[i];
+      for (int i = 0; i < W; ++i) {
+        lo += i < wave ? s_scan[i] : 0;
+        first += s_scan[i];
+        C += s_scan[i] + s_rest[i];
+      }
     }
-    C = first;
-    if (nf > NTHR)
-      for (int i = 0; i < W; ++i) C += s_rest[i];
     const int U = C * LK;  // the host sends calls of 2^30 stages or more to whole row groups
     per1 = a.pf_w1 ? max((U + a.pf_w1 - 1) / a.pf_w1, a.pf_min1) : 0;
     per2 = max((U + a.pf_w2 - 1) / a.pf_w2, a.pf_min2);
@@ -167,28 +175,33 @@ void prefill_kernel(AttnArgs a, int layers) {
     if (u < uend) {  // workgroup-uniform
       pos.lk = u / C;
       const int rem = u - pos.lk * C;
-      for (int base = 0;;) {
-        if (rem >= lo && rem < lo + v) {
-          s_pos[0] = base + tid;
-          s_pos[1] = lo;
-        }
-        if (rem < first) break;  // workgroup-uniform
-        base += NTHR;
-        v = base + tid < nf ? weight_of(base + tid) : 0;
-        inc = wave_scan(v);
-        __syncthreads();
-        if (lane == 63) s_scan[wave] = inc;
-        __syncthreads();
-        lo = first + inc - v;
+      if (few) {
+        pos.f = __popcll(__ballot(lane < nf && inc <= rem));
+        pos.start = pos.lk * C + __builtin_amdgcn_readlane(lo, pos.f);
+      } else {
+        for (int base = 0;;) {
+          if (rem >= lo && rem < lo + v) {
+            s_pos[0] = base + tid;
+            s_pos[1] = lo;
+          }
+          if (rem < first) break;  // workgroup-uniform
+          base += NTHR;
+          v = base + tid < nf ? weight_of(base + tid) : 0;
+          inc = wave_scan(v);
+          __syncthreads();
+          if (lane == 63) s_scan[wave] = inc;
+          __syncthreads();
+          lo = first + inc - v;
 #pragma unroll
-        for (int i = 0; i < W; ++i) {
-          lo += i < wave ? s_scan[i] : 0;
-          first += s_scan[i];
+          for (int i = 0; i < W; ++i) {
+            lo += i < wave ? s_scan[i] : 0;
+            first += s_scan[i];
+          }
         }
+        __syncthreads();
+        pos.f = __builtin_amdgcn_readfirstlane(s_pos[0]);
+        pos.start = pos.lk * C + __builtin_amdgcn_readfirstlane(s_pos[1]);
       }
-      __syncthreads();
-      pos.f = __builtin_amdgcn_readfirstlane(s_pos[0]);
-      pos.start = pos.lk * C + __builtin_amdgcn_readfirstlane(s_pos[1]);
       pos.wt = __builtin_amdgcn_readfirstlane(weight_of(pos.f));
     }
   }
@@ -246,15 +259,14 @@ void prefill_kernel(AttnArgs a, int layers) {
       int id[kPfIds / NTHR];
 #pragma unroll
       for (int i = 0; i < kPfIds / NTHR; ++i) id[i] = i * NTHR + tid < nids ? btrow[max(0, min(blk0 + i * NTHR + tid, nbk - 1))] : -1;
+      ++window;
       __syncthreads();  // the ids before these are no longer read
-      if (tid == 0) s_bad = 0;
-      __syncthreads();
 #pragma unroll
       for (int i = 0; i < kPfIds / NTHR; ++i) {
         const int j = i * NTHR + tid;
         if (j < nids) {
           const bool in = blk0 + j < nbk, ok = in && id[i] >= 0 && id[i] < a.num_blocks;
-          if (in && !ok) s_bad = 1;
+          if (in && !ok) s_bad = window;
           lpb[j] = ok ? id[i] : -1;
         }
       }
@@ -288,223 +300,223 @@ void prefill_kernel(AttnArgs a, int layers) {
     float m_run = -INFINITY, l_run = 0.0f;  // pass 1
     bool slow = false;                      // pass 1: every stage through the online update
     for (;;) {
-    if constexpr (OUT) {
+      if constexpr (OUT) {
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) acc[dt] = (f32x16)0.0f;
-    }
-    for (int wlo = slo; wlo < shi; wlo += kPfIds / 4) {  // page-id windows; workgroup-uniform
-      const int nit = min(kPfIds / 4, shi - wlo);        // stages in the window
-      if (wlo > slo) stage_ids(wlo);
-      const int bad = __builtin_amdgcn_readfirstlane(s_bad);
-      // units of the window (32 keys): x = 0 .. 2 nit - 1, the first at key 32 * ux0
-      const int ux0 = 2 * wlo, nx = 2 * nit;
-      const uint4* vh_grp = a.vhat + (int64_t)grp * a.vh_stages * (DT * 128) + lane;
-      // The loop multiplies q.k^T one unit ahead of the scores and p.V one unit behind them:
-      // buffer s holds K of units 2s + 1, 2s + 2 and V of units 2s - 1, 2s.  Past the window's
-      // ends the nearest unit is loaded; its products are not used, or meet p = 0.
-      int id[NK / W];   // page ids of the next fetch
-      uint4 stg[CPW];   // this wavefront's chunks of the next stage
-      auto next_ids = [&](int s) {
+        for (int dt = 0; dt < DT; ++dt) acc[dt] = (f32x16)0.0f;
+      }
+      for (int wlo = slo; wlo < shi; wlo += kPfIds / 4) {  // page-id windows; workgroup-uniform
+        const int nit = min(kPfIds / 4, shi - wlo);        // stages in the window
+        if (wlo > slo) stage_ids(wlo);
+        const bool bad = __builtin_amdgcn_readfirstlane(s_bad) == window;  // an invalid id in the window
+        // units of the window (32 keys): x = 0 .. 2 nit - 1, the first at key 32 * ux0
+        const int ux0 = 2 * wlo, nx = 2 * nit;
+        const uint4* vh_grp = a.vhat + (int64_t)grp * a.vh_stages * (DT * 128) + lane;
+        // The loop multiplies q.k^T one unit ahead of the scores and p.V one unit behind them:
+        // buffer s holds K of units 2s + 1, 2s + 2 and V of units 2s - 1, 2s.  Past the window's
+        // ends the nearest unit is loaded; its products are not used, or meet p = 0.
+        int id[NK / W];   // page ids of the next fetch
+        uint4 stg[CPW];   // this wavefront's chunks of the next stage
+        auto next_ids = [&](int s) {
 #pragma unroll
-        for (int j = 0; j < NK / W; ++j) {
-          const int c = j * W + wave, x = min(max(2 * s + 1 + c / CU, 0), nx - 1);
-          id[j] = lpb[2 * x + (c % CU) / PU];
-        }
-      };
-      auto fetch1 = [&](int s, int j) {  // chunk j * W + wave of stage s
-        const int c = j * W + wave;
-        if (j < NK / W) {
-          const int64_t pg = max(__builtin_amdgcn_readfirstlane(id[j]), 0);
-          return load_stream16(klayer + pg * kpage + (c % PU) * 512 + lane * 8);
-        }
-        const int cc = c - NK, x = min(max(2 * s - 1 + cc / CU, 0), nx - 1);
-        const int blk = min(2 * (ux0 + x) + (cc % CU) / PU, 2 * a.vh_stages - 1);
-        return vh_grp[(int64_t)blk * (DT * 64) + (cc % PU) * 64];
-      };
-      auto stash1 = [&](uint4* buf, int j) { buf[(j * W + wave) * 64 + lane] = stg[j]; };
-      auto publish = [&]() {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-      };
-      // The wavefront's iterations: those of fully visible stages, then those that need the mask
-      // (pass 1: the first stage too, whose maximum the fast ones start from).
-      const int nfast = !active || bad || slow ? 0 : min(nit, max(0, (ufull - ux0) >> 1));
+          for (int j = 0; j < NK / W; ++j) {
+            const int c = j * W + wave, x = min(max(2 * s + 1 + c / CU, 0), nx - 1);
+            id[j] = lpb[2 * x + (c % CU) / PU];
+          }
+        };
+        auto fetch1 = [&](int s, int j) {  // chunk j * W + wave of stage s
+          const int c = j * W + wave;
+          if (j < NK / W) {
+            const int64_t pg = max(__builtin_amdgcn_readfirstlane(id[j]), 0);
+            return load_stream16(klayer + pg * kpage + (c % PU) * 512 + lane * 8);
+          }
+          const int cc = c - NK, x = min(max(2 * s - 1 + cc / CU, 0), nx - 1);
+          const int blk = min(2 * (ux0 + x) + (cc % CU) / PU, 2 * a.vh_stages - 1);
+          return vh_grp[(int64_t)blk * (DT * 64) + (cc % PU) * 64];
+        };
+        auto stash1 = [&](uint4* buf, int j) { buf[(j * W + wave) * 64 + lane] = stg[j]; };
+        auto publish = [&]() {
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+          __builtin_amdgcn_s_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        };
+        // The wavefront's iterations: those of fully visible stages, then those that need the mask
+        // (pass 1: the first stage too, whose maximum the fast ones start from).
+        const int nfast = !active || bad || slow ? 0 : min(nit, max(0, (ufull - ux0) >> 1));
 
-      // One iteration is 2 units x NM steps.  A step issues one MFMA -- q.k^T of the next unit,
-      // and in pass 2 p.V of the one before in turn -- reads the LDS operand of the step kAhead
-      // later and works on 16 / NM scores of this unit.  The three do not depend on each other,
-      // and the scheduling barriers hold the order: an MFMA takes 32 cycles of the matrix unit, a
-      // score about as many of the VALU.  The first steps also write a chunk each of the next
-      // stage, whose loads went out an iteration ago, to the third buffer, and send the loads of
-      // the stage after it; the iteration's one barrier, at the end of the first unit, publishes
-      // the stage, so that the operand reads run on across iterations.
-      constexpr int NM = OUT ? KS + 2 * DT : KS, SPM = 16 / NM, kAhead = OUT ? 4 : 2;
-      constexpr int MS = (CPW + 1) & ~1;  // the steps that write and load chunks
-      static_assert(CPW <= NM / 2, "kLater operand reads lie between the chunk writes and the barrier");
-      constexpr int kLater = NM - MS < NM / 2 ? NM - MS : NM / 2;
-      static_assert(KS == 2 * DT && NM * SPM == 16, "q.k^T and p.V steps alternate");
-      uint4 *cur = ring[0], *nxt = ring[1], *third = ring[2];
-      auto operand = [&](const uint4* sb, int m) {  // step m: of unit m / NM, k step or tile i
-        const int un = m / NM, i = OUT ? (m % NM) / 2 : m % NM;
-        const char* kb = reinterpret_cast<const char*>(sb) + kofs;
-        return OUT && (m & 1) ? __builtin_bit_cast(bf16x8, sb[(NK + un * CU + i) * 64 + lane])
-                              : *reinterpret_cast<const bf16x8*>(kb + un * (CU * 1024) + i * 512);
-      };
-      bf16x8 op[kAhead];
-      f32x16 sc;        // products of the unit whose scores come next
-      uint32_t pw[8];   // p of the unit whose p.V product comes next: two MFMA operands
-      auto pop = [&](int h) {
-        return __builtin_bit_cast(bf16x8, make_uint4(pw[4 * h], pw[4 * h + 1], pw[4 * h + 2], pw[4 * h + 3]));
-      };
-      auto body = [&](int it, bool mask) {
-        next_ids(it + 2);
-        f32x16 sn = (f32x16)0.0f;
-        uint32_t pn[8];
-        float last = 0.0f, nm = OUT ? nml : -m_run * kLog2e;
-        float y[16];
+        // One iteration is 2 units x NM steps.  A step issues one MFMA -- q.k^T of the next unit,
+        // and in pass 2 p.V of the one before in turn -- reads the LDS operand of the step kAhead
+        // later and works on 16 / NM scores of this unit.  The three do not depend on each other,
+        // and the scheduling barriers hold the order: an MFMA takes 32 cycles of the matrix unit, a
+        // score about as many of the VALU.  The first steps also write a chunk each of the next
+        // stage, whose loads went out an iteration ago, to the third buffer, and send the loads of
+        // the stage after it; the iteration's one barrier, at the end of the first unit, publishes
+        // the stage, so that the operand reads run on across iterations.
+        constexpr int NM = OUT ? KS + 2 * DT : KS, SPM = 16 / NM, kAhead = OUT ? 4 : 2;
+        constexpr int MS = (CPW + 1) & ~1;  // the steps that write and load chunks
+        static_assert(CPW <= NM / 2, "kLater operand reads lie between the chunk writes and the barrier");
+        constexpr int kLater = NM - MS < NM / 2 ? NM - MS : NM / 2;
+        static_assert(KS == 2 * DT && NM * SPM == 16, "q.k^T and p.V steps alternate");
+        uint4 *cur = ring[0], *nxt = ring[1], *third = ring[2];
+        auto operand = [&](const uint4* sb, int m) {  // step m: of unit m / NM, k step or tile i
+          const int un = m / NM, i = OUT ? (m % NM) / 2 : m % NM;
+          const char* kb = reinterpret_cast<const char*>(sb) + kofs;
+          return OUT && (m & 1) ? __builtin_bit_cast(bf16x8, sb[(NK + un * CU + i) * 64 + lane])
+                                : *reinterpret_cast<const bf16x8*>(kb + un * (CU * 1024) + i * 512);
+        };
+        bf16x8 op[kAhead];
+        f32x16 sc;        // products of the unit whose scores come next
+        uint32_t pw[8];   // p of the unit whose p.V product comes next: two MFMA operands
+        auto pop = [&](int h) {
+          return __builtin_bit_cast(bf16x8, make_uint4(pw[4 * h], pw[4 * h + 1], pw[4 * h + 2], pw[4 * h + 3]));
+        };
+        auto body = [&](int it, bool mask) {
+          next_ids(it + 2);
+          f32x16 sn = (f32x16)0.0f;
+          uint32_t pn[8];
+          float last = 0.0f, nm = OUT ? nml : -m_run * kLog2e;
+          float y[16];
 #pragma unroll
-        for (int m = 0; m < 2 * NM; ++m) {
-          const int un = m / NM, mm = m % NM, i = OUT ? mm / 2 : mm;
-          if (OUT && (m & 1))
-            acc[i % DT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op[m % kAhead], pop(i / DT), acc[i % DT], 0, 0, 0);
-          else
-            sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op[m % kAhead], qop[i], mm == 0 ? (f32x16)0.0f : sn, 0, 0, 0);
-          op[m % kAhead] = m + kAhead < 2 * NM ? operand(cur, m + kAhead) : operand(nxt, m + kAhead - 2 * NM);
-          // lane (g, n), score e: key 8 (e / 4) + 4 g + e % 4 of the unit
-          int limb[2];
-          if (mask) {
+          for (int m = 0; m < 2 * NM; ++m) {
+            const int un = m / NM, mm = m % NM, i = OUT ? mm / 2 : mm;
+            if (OUT && (m & 1))
+              acc[i % DT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op[m % kAhead], pop(i / DT), acc[i % DT], 0, 0, 0);
+            else
+              sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op[m % kAhead], qop[i], mm == 0 ? (f32x16)0.0f : sn, 0, 0, 0);
+            op[m % kAhead] = m + kAhead < 2 * NM ? operand(cur, m + kAhead) : operand(nxt, m + kAhead - 2 * NM);
+            // lane (g, n), score e: key 8 (e / 4) + 4 g + e % 4 of the unit
+            int limb[2];
+            if (mask) {
 #pragma unroll
-            for (int h = 0; h < 2; ++h) limb[h] = lpb[2 * (2 * it + un) + h] >= 0 ? lim - 32 * (ux0 + 2 * it + un) - 4 * g : -1;
-          }
-#pragma unroll
-          for (int e = mm * SPM; e < (mm + 1) * SPM; ++e) {
-            float v = eager(sc[e]);
-            if (mask) v = 8 * (e >> 2) + (e & 3) <= limb[e >> 3] ? v : -INFINITY;
-            if (!OUT && mask) {
-              y[e] = v;
-              continue;
+              for (int h = 0; h < 2; ++h) limb[h] = lpb[2 * (2 * it + un) + h] >= 0 ? lim - 32 * (ux0 + 2 * it + un) - 4 * g : -1;
             }
-            const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(v, kExpCoef, nm));
-            if (OUT) {
-              if (e & 1)
-                pn[e / 2] = pack_bf16x2(last, p);
-              else
-                last = p;
-            } else {
-              y[e & 3] = e < 4 ? p : y[e & 3] + p;
-            }
-          }
-          if (m < CPW) {
-            stash1(nxt, m);
-            stg[m] = fetch1(it + 2, m);
-          }
-          if (SPM > 1 || (m & 1)) __builtin_amdgcn_sched_barrier(0);
-          if (m == MS - 1) asm volatile("" ::: "memory");
-          if (m == NM - 1) {
-            // LDS operations of a wavefront complete in order: with at most kLater outstanding, all
-            // issued after the writes (the operand reads of steps MS .. NM - 1), the writes are done
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_s_waitcnt(0xC07F | (kLater << 8));
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_sched_barrier(0);
-          }
-          if (mm == NM - 1) {
-            sc = sn;
-            if constexpr (OUT) {
 #pragma unroll
-              for (int w = 0; w < 8; ++w) pw[w] = pn[w];
-            } else {
-#pragma clang fp contract(off)
-              if (mask) {
-                // Online (max, sum) per lane: the running sum rescaled by
-                // exp2((m_old - m_new) log2 e), which is exactly 1 while the max stays (the one-FMA
-                // form exp2(m_old log2 e - RN(m_new log2 e)) is off by the product's rounding on
-                // every update, and L drifted by ~1e-5 at T = 8192: rel-L2 7e-4 against eager)
-                float mt = -INFINITY;
-#pragma unroll
-                for (int w = 0; w < 16; w += 2) mt = max3f(mt, y[w], y[w + 1]);
-                mt *= kUnit;
-                if (mt != -INFINITY) {
-                  const float mn = fmaxf(m_run, mt);
-                  const float f = __builtin_amdgcn_exp2f((m_run - mn) * kLog2e);
-                  nm = -mn * kLog2e;
-#pragma unroll
-                  for (int w = 0; w < 16; ++w) y[w] = __builtin_amdgcn_exp2f(__builtin_fmaf(y[w], kExpCoef, nm));
-#pragma unroll
-                  for (int w = 4; w < 16; ++w) y[w & 3] = y[w & 3] + y[w];
-                  l_run = l_run * f + ((y[0] + y[1]) + (y[2] + y[3]));
-                  m_run = mn;
-                }
+            for (int e = mm * SPM; e < (mm + 1) * SPM; ++e) {
+              float v = eager(sc[e]);
+              if (mask) v = 8 * (e >> 2) + (e & 3) <= limb[e >> 3] ? v : -INFINITY;
+              if (!OUT && mask) {
+                y[e] = v;
+                continue;
+              }
+              const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(v, kExpCoef, nm));
+              if (OUT) {
+                if (e & 1)
+                  pn[e / 2] = pack_bf16x2(last, p);
+                else
+                  last = p;
               } else {
-                l_run = l_run + ((y[0] + y[1]) + (y[2] + y[3]));
+                y[e & 3] = e < 4 ? p : y[e & 3] + p;
+              }
+            }
+            if (m < CPW) {
+              stash1(nxt, m);
+              stg[m] = fetch1(it + 2, m);
+            }
+            if (SPM > 1 || (m & 1)) __builtin_amdgcn_sched_barrier(0);
+            if (m == MS - 1) asm volatile("" ::: "memory");
+            if (m == NM - 1) {
+              // LDS operations of a wavefront complete in order: with at most kLater outstanding, all
+              // issued after the writes (the operand reads of steps MS .. NM - 1), the writes are done
+              asm volatile("" ::: "memory");
+              __builtin_amdgcn_s_waitcnt(0xC07F | (kLater << 8));
+              __builtin_amdgcn_s_barrier();
+              asm volatile("" ::: "memory");
+              __builtin_amdgcn_sched_barrier(0);
+            }
+            if (mm == NM - 1) {
+              sc = sn;
+              if constexpr (OUT) {
+#pragma unroll
+                for (int w = 0; w < 8; ++w) pw[w] = pn[w];
+              } else {
+#pragma clang fp contract(off)
+                if (mask) {
+                  // Online (max, sum) per lane: the running sum rescaled by
+                  // exp2((m_old - m_new) log2 e), which is exactly 1 while the max stays (the one-FMA
+                  // form exp2(m_old log2 e - RN(m_new log2 e)) is off by the product's rounding on
+                  // every update, and L drifted by ~1e-5 at T = 8192: rel-L2 7e-4 against eager)
+                  float mt = -INFINITY;
+#pragma unroll
+                  for (int w = 0; w < 16; w += 2) mt = max3f(mt, y[w], y[w + 1]);
+                  mt *= kUnit;
+                  if (mt != -INFINITY) {
+                    const float mn = fmaxf(m_run, mt);
+                    const float f = __builtin_amdgcn_exp2f((m_run - mn) * kLog2e);
+                    nm = -mn * kLog2e;
+#pragma unroll
+                    for (int w = 0; w < 16; ++w) y[w] = __builtin_amdgcn_exp2f(__builtin_fmaf(y[w], kExpCoef, nm));
+#pragma unroll
+                    for (int w = 4; w < 16; ++w) y[w & 3] = y[w & 3] + y[w];
+                    l_run = l_run * f + ((y[0] + y[1]) + (y[2] + y[3]));
+                    m_run = mn;
+                  }
+                } else {
+                  l_run = l_run + ((y[0] + y[1]) + (y[2] + y[3]));
+                }
               }
             }
           }
-        }
-        uint4* const t = cur;
-        cur = nxt;
-        nxt = third;
-        third = t;
-      };
-
-      // stage 0 and unit 0's K (slot 1 of stage -1), loaded together
-      uint4 stg0[NK / W];
-      next_ids(-1);
-#pragma unroll
-      for (int j = 0; j < NK / W; ++j) stg0[j] = fetch1(-1, j);
-      next_ids(0);
-#pragma unroll
-      for (int j = 0; j < CPW; ++j) stg[j] = fetch1(0, j);
-      next_ids(1);
-#pragma unroll
-      for (int j = 0; j < NK / W; ++j) third[(j * W + wave) * 64 + lane] = stg0[j];
-#pragma unroll
-      for (int j = 0; j < CPW; ++j) {
-        stash1(cur, j);
-        stg[j] = fetch1(1, j);
-      }
-      publish();
-      {
-        const char* kb = reinterpret_cast<const char*>(third) + CU * 1024 + kofs;
-        sc = (f32x16)0.0f;
-#pragma unroll
-        for (int kk = 0; kk < KS; ++kk)
-          sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(kb + kk * 512), qop[kk], sc, 0, 0, 0);
-#pragma unroll
-        for (int w = 0; w < 8; ++w) pw[w] = 0;
-#pragma unroll
-        for (int m = 0; m < kAhead; ++m) op[m] = operand(cur, m);
-      }
-      int it = 0;
-      if (!OUT && active) body(it++, true);
-      for (; it < nfast; ++it) body(it, false);
-      if (active) {
-        for (; it < nit; ++it) body(it, true);
-      } else {  // a wavefront without rows loads its share
-        for (; it < nit; ++it) {
-          next_ids(it + 2);
-#pragma unroll
-          for (int j = 0; j < CPW; ++j) {
-            stash1(nxt, j);
-            stg[j] = fetch1(it + 2, j);
-          }
-          publish();
           uint4* const t = cur;
           cur = nxt;
           nxt = third;
           third = t;
-        }
-      }
-      if constexpr (OUT) {  // the last unit's p.V
-        if (active) {
+        };
+
+        // stage 0 and unit 0's K (slot 1 of stage -1), loaded together
+        uint4 stg0[NK / W];
+        next_ids(-1);
 #pragma unroll
-          for (int i = 0; i < 2 * DT; ++i)
-            acc[i % DT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(operand(cur, 2 * i + 1), pop(i / DT), acc[i % DT], 0, 0, 0);
+        for (int j = 0; j < NK / W; ++j) stg0[j] = fetch1(-1, j);
+        next_ids(0);
+#pragma unroll
+        for (int j = 0; j < CPW; ++j) stg[j] = fetch1(0, j);
+        next_ids(1);
+#pragma unroll
+        for (int j = 0; j < NK / W; ++j) third[(j * W + wave) * 64 + lane] = stg0[j];
+#pragma unroll
+        for (int j = 0; j < CPW; ++j) {
+          stash1(cur, j);
+          stg[j] = fetch1(1, j);
+        }
+        publish();
+        {
+          const char* kb = reinterpret_cast<const char*>(third) + CU * 1024 + kofs;
+          sc = (f32x16)0.0f;
+#pragma unroll
+          for (int kk = 0; kk < KS; ++kk)
+            sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(kb + kk * 512), qop[kk], sc, 0, 0, 0);
+#pragma unroll
+          for (int w = 0; w < 8; ++w) pw[w] = 0;
+#pragma unroll
+          for (int m = 0; m < kAhead; ++m) op[m] = operand(cur, m);
+        }
+        int it = 0;
+        if (!OUT && active) body(it++, true);
+        for (; it < nfast; ++it) body(it, false);
+        if (active) {
+          for (; it < nit; ++it) body(it, true);
+        } else {  // a wavefront without rows loads its share
+          for (; it < nit; ++it) {
+            next_ids(it + 2);
+#pragma unroll
+            for (int j = 0; j < CPW; ++j) {
+              stash1(nxt, j);
+              stg[j] = fetch1(it + 2, j);
+            }
+            publish();
+            uint4* const t = cur;
+            cur = nxt;
+            nxt = third;
+            third = t;
+          }
+        }
+        if constexpr (OUT) {  // the last unit's p.V
+          if (active) {
+#pragma unroll
+            for (int i = 0; i < 2 * DT; ++i)
+              acc[i % DT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(operand(cur, 2 * i + 1), pop(i / DT), acc[i % DT], 0, 0, 0);
+          }
         }
       }
-    }
       if constexpr (OUT) {
         break;
       } else {

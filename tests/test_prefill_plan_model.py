@@ -12,7 +12,7 @@ import pytest
 
 from specdec_amd import _native
 
-WAVES, ROWS, STAGE, SEG, MIN, CUS = 8, 256, 64, 2, 4, 256
+ROWS, STAGE, SEG, MIN, CUS = 256, 64, 6, 3, 256
 SYNC_PART, DESC, MAX_GROUPS = 8 << 20, (1 << 14) * 8, 1 << 14
 
 
@@ -53,7 +53,7 @@ def plan(groups, r, s, g, d, t):
         return total, 0, 0, MIN, split, slots, False, have
     w1, min1 = 0, MIN
     if split >= 2:
-        w1 = min(2 * CUS, cdiv(u, MIN))
+        w1 = min(CUS, cdiv(u, MIN))
         min1 = max(min1, cdiv(stages(nrg - 1, s, g, t) - 1, split - 1))
     return total, w1, w2, min1, split, slots, w2 + n <= have, have
 
