@@ -34,7 +34,7 @@
 // (head_dim 128; MFMA 2,048).  Measured, both passes, of one KV pair's 2048 rows x 8192 keys
 // (12/2/128, 14/2/64), 777 x 5000 (14/2/64), 2048 x 2048 and 300 x 5000 (12/2/128), before (16x16
 // MFMAs, a row group's rows of one head, parts per row group) and now:
-//   233 -> 183, 152 -> 122, 83 -> 56, 77 -> 61, 74 -> 54 us.
+//   233 -> 175, 152 -> 120, 83 -> 50, 77 -> 57, 74 -> 50 us.
 // What it took: one wave's LDS operand reads run across the stage barrier (three buffers, waits
 // counted by hand: 92 -> 80 us of pass 2's loop), the parts' sum in its own launch (the last part
 // to finish summing 470 KB alone held the end up by 29 us), q.k^T, scores and p.V of three units
@@ -165,10 +165,14 @@ void prefill_kernel(AttnArgs a, int layers) {
     const int U = C * LK;  // the host sends calls of 2^30 stages or more to whole row groups
     per1 = a.pf_w1 ? max((U + a.pf_w1 - 1) / a.pf_w1, a.pf_min1) : 0;
     per2 = max((U + a.pf_w2 - 1) / a.pf_w2, a.pf_min2);
-    // consecutive ranges on one XCD (workgroup w runs on XCD w mod 8), so that an XCD's L2 holds
-    // the K and V of few KV heads
+    // Consecutive ranges on one XCD (workgroup i runs on XCD i mod 8), so that an XCD's L2 holds
+    // the K and V of few KV heads -- where those of all do not fit its 4 MiB (BF16 K and
+    // dequantized V, 4 bytes a dimension).  Where they fit, ranges in launch order are faster
+    // (777 x 5000 of 14/2/64 53 against 50 us, 2048 x 2048 of 12/2/128 60 against 57; 1500 x 12000 of
+    // 14/2/64, 6 MiB: 133 against 135).
     const int nw = (int)gridDim.x, q8 = nw >> 3, r8 = nw & 7, xcd = (int)blockIdx.x & 7;
-    const int w = xcd * q8 + min(xcd, r8) + ((int)blockIdx.x >> 3);
+    const bool large = (int64_t)LK * a.B * a.max_seq_len * (4 * D) > (4 << 20);
+    const int w = large ? xcd * q8 + min(xcd, r8) + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
     const int per = OUT ? per2 : per1;
     u = min(w * per, U);
     uend = min(u + per, U);
@@ -327,7 +331,9 @@ void prefill_kernel(AttnArgs a, int layers) {
           const int c = j * W + wave;
           if (j < NK / W) {
             const int64_t pg = max(__builtin_amdgcn_readfirstlane(id[j]), 0);
-            return load_stream16(klayer + pg * kpage + (c % PU) * 512 + lane * 8);
+            // cached, unlike the other kernels' K: every row group reads it again (2048 x 8192 of
+          // 12/2/128 183 us with the streaming hint, 175 without)
+          return *reinterpret_cast<const uint4*>(klayer + pg * kpage + (c % PU) * 512 + lane * 8);
           }
           const int cc = c - NK, x = min(max(2 * s - 1 + cc / CU, 0), nx - 1);
           const int blk = min(2 * (ux0 + x) + (cc % CU) / PU, 2 * a.vh_stages - 1);
