@@ -479,7 +479,7 @@ def prefill_row(torch, dev, h, kv, d, s, t, ref, nrep=2):
     flops = 4 * h * keys * d                         # q.k^T and p.V, as the eager path computes them
     executed = 6 * h * keys * d                      # pass 1 recomputes q.k^T
     return {"q_heads": h, "kv_heads": kv, "head_dim": d, "q_rows": s, "keys": t, "us_per_call": round(us, 1),
-            "launches": 2, "workspace_MiB": round(nbytes / 2 ** 20, 2),
+            "launches": 3, "workspace_MiB": round(nbytes / 2 ** 20, 2),
             "transient_MiB_workspace_plus_output": round(transient / 2 ** 20, 2),
             "TFLOPs_algorithmic": round(flops / (us * 1e-6) / 1e12, 1),
             "TFLOPs_executed": round(executed / (us * 1e-6) / 1e12, 1),

@@ -14,7 +14,8 @@
 //                 large for one launch);
 //   group_kernel  256 or more one-tile groups the single launch cannot hold: persistent
 //                 workgroups that each compute whole groups;
-//   prefill_kernel many query rows (prefill chunks), two passes;
+//   prefill_kernel many query rows (prefill chunks), two passes and the sum of their parts
+//                 (sdv_prefill.h);
 // and the three launches, for the rest and for the profiling split (phase_mask):
 //
 //   qk_kernel     workgroup = 4 wavefronts = one chunk of page blocks of one (layer*batch,
@@ -2352,7 +2353,7 @@ static bool try_fused_per_layer(const AttnArgs& a, int layers, hipStream_t st) {
 // and the caller appends with the append kernel and calls again without a.app_v.
 template <int D>
 static bool launch_all(const AttnArgs& a, const Plan& p, int zdim, hipStream_t st, int phases) {
-  if (p.n_row_groups > 1) {  // many query rows: the two prefill passes
+  if (p.n_row_groups > 1) {  // many query rows: the two prefill passes and the parts' sum
     if (a.app_v) return false;
     const int layers = zdim / a.B;
     const unsigned whole = (unsigned)(p.groups * p.pf_nrg);

@@ -1,12 +1,13 @@
 // Prefill rows: shapes with more query rows than one row-tile group holds (R = G*S > 64: prefill
-// and chunked-prefill blocks, model_self.py:471-504, 637-648) in two launches.
+// and chunked-prefill blocks, model_self.py:471-504, 637-648) in two passes and a launch that
+// sums the parts of pass 2.
 // Included by sdv_attn.hip, which defines AttnArgs, the synchronisation area and the helpers.
 //
 //   pass 1  S^T = K Q^T on MFMA, scores rounded to BF16 as the eager path does, offset-causal
 //           mask, online (max, sum) per row.  Also dequantizes V once, in the lane order of pass
 //           2's MFMA operand.
 //   pass 2  recomputes the scores, forms p = bf16(exp(s - M) / L) from pass 1's statistics and
-//           accumulates O^T = V_hat^T P^T on MFMA.
+//           accumulates O^T = V_hat^T P^T on MFMA; a third launch sums its parts.
 //
 // Rows are token-major (row r: token r / G, head r % G), so the rows of a group of 256 see nearly
 // the same keys.  Row r sees keys j <= T - S + r / G (the eager mask); a row that sees no key

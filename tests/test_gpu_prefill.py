@@ -77,9 +77,8 @@ def test_prefill_chunk_draft_2048x8192(cuda_device):
                                      (12, 128, 11, 40000), (12, 128, 1000, 1000), (14, 64, 11, 270000)])
 def test_prefill_shapes(cuda_device, h, d, s, t):
     """A first chunk from an empty cache (T = S, triangular mask), odd sizes, short blocks over
-    long contexts and S not a multiple of 16.  A workgroup stages 256 page ids in LDS at a time:
-    at T = 270,000 (16,875 blocks) every pass-1 key part (of 64) spans two such windows and every
-    pass-2 part (of 8) nine, so both passes cross windows with stages in flight."""
+    long contexts and S not a multiple of 16; at T = 270,000 (4,219 stages of 64 keys for each of
+    two row groups) pass 1's statistics hold 64 segments per row."""
     announce(f"prefill {h}/2/{d} S={s} T={t}")
     _prefill_case(cuda_device, h, 2, d, s, t, seed=710 + s + t, chunk_rows=512)
 
@@ -87,8 +86,8 @@ def test_prefill_shapes(cuda_device, h, d, s, t):
 @pytest.mark.parametrize("s,h,d", [(96, 12, 128), (256, 12, 128), (256, 14, 64)])
 def test_prefill_ragged_batch_token_major(cuda_device, s, h, d):
     """Two sequences of different lengths in one call, q in the projection layout (B, S, H, D).
-    With S a multiple of pass 2's 128 rows (S = 256) pass 2's parts follow each row group's key
-    count, planned for the longest sequence: the shorter one's row groups leave parts empty."""
+    The launches are sized for the longest sequence and the ranges of stages cut from the
+    actual lengths; S = 256 takes the workspace of S a multiple of 128."""
     announce(f"prefill ragged batch, token-major q, S={s} {h}/2/{d}")
     g = wl.gen(720 + s + d, cuda_device)
     lens, kv = [3000, 700], 2
@@ -113,8 +112,7 @@ def test_prefill_ragged_batch_token_major(cuda_device, s, h, d):
 def test_prefill_multi_layer_call(cuda_device):
     """Two layers x two ragged sequences of 128 new rows in one call (q in the projection layout
     (L, B, S, H, D)): every (layer, sequence) pair has its own pass-1 statistics, dequantized V
-    and pass-2 parts (by key count: S is a multiple of 128), and each output is within the bar
-    of the eager reference."""
+    and pass-2 parts, and each output is within the bar of the eager reference."""
     announce("prefill 2 layers x 2 ragged sequences, S=128, one call")
     g = wl.gen(725, cuda_device)
     L, lens, s, h, kv, d = 2, [2500, 900], 128, 12, 2, 128
@@ -154,10 +152,9 @@ def test_prefill_deterministic(cuda_device):
 
 @pytest.mark.parametrize("h,d,s", [(14, 64, 300), (12, 128, 300), (12, 128, 256)])
 def test_prefill_key_parts_repeat_and_replay(cuda_device, h, d, s):
-    """Pass 2 splits each row group's keys in parts, and the part that finishes last sums them
-    (a per-row-group counter that it zeroes again): repeated eager calls and the replays of a
-    recorded call -- which reuse one tag -- with eager calls between them are bitwise equal, on
-    a batch of two sequences (two counters per KV head); S = 256 takes the parts by key count."""
+    """Row groups that several workgroups' ranges cut leave their parts in slots, which a third
+    launch sums: repeated eager calls and the replays of a recorded call -- which reuse one tag -- with eager calls between them are bitwise equal, on
+    a batch of two sequences; S = 256 takes the workspace of S a multiple of 128."""
     announce(f"prefill {h}/2/{d} S={s} key parts: repeats and graph replays")
     g = wl.gen(740 + d + s, cuda_device)
     lens, kv = [3000, 1200], 2

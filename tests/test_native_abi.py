@@ -205,12 +205,10 @@ def _round256(x):
 
 def test_prefill_workspace_follows_the_part_plan(lib):
     """The prefill workspace is the synchronisation prefix, pass 1's (max, sum) per row and key
-    part, pass 2's fp32 part slots (128 rows per row group, as many slots as its most-split row
-    group) and V dequantized once (one 1 KiB tile per 16 dimensions and two blocks).  2048 x 8192
-    (12/2/128): pass 1 in 8 parts (1,536 workgroups of 128 rows), pass 2 by key count, at most 3
-    parts (the last 10 of each head's 16 row groups); with S not a multiple of 128 (S = T =
-    1000) pass 1 takes 7 parts (no fewer than 8 blocks each) and pass 2 splits every row group
-    alike, in 5."""
+    part, pass 2's fp32 part slots and V dequantized once (one 1 KiB tile per 16 dimensions and
+    two blocks), by a fixed rule that the launches' split is fitted to.  2048 x 8192 (12/2/128):
+    statistics of 8 parts per row, three slots per 128 rows; S = T = 1000 (not a multiple of 128):
+    7 parts, five slots."""
     H, KV, D, S, T = 12, 2, 128, 2048, 8192
     R, groups = H // KV * S, KV
     want = (_native.SYNC_BYTES + _round256(groups * R * 8 * 8) + _round256(groups * (R // 128) * 3 * 128 * D * 4)

@@ -123,9 +123,9 @@ def _batch_cache(dev, layers, kv, d, lens, seed):
 
 def test_noalloc_group_and_prefill_paths(cuda_device):
     """The per-group kernel (a claim counter that its last workgroup resets) and the head_dim 64
-    prefill (a counter per row group that the last key part resets) through the scratch, in the
-    order group -> prefill -> smaller group -> prefill again -> prefill whose pass-2 parts
-    follow each row group's key count: every call equals sdv_paged_attention's output bit for
+    prefill (part slots in the scratch's partials too) through the scratch, in the
+    order group -> prefill -> smaller group -> prefill again -> prefill whose S is a multiple of
+    128: every call equals sdv_paged_attention's output bit for
     bit."""
     lib = _native.load()
     g = wl.gen(920, cuda_device)
