@@ -86,6 +86,15 @@ __device__ __forceinline__ int wave_scan(int v) {
   return v;
 }
 
+// Bound of pass 1's sums of exponentials in the fully visible stages, whose exponents are taken
+// against an earlier maximum: a unit that would bring a lane's sum to this much goes through the
+// online update instead.  The two lanes of a row and its segments (at most 64) can then be added
+// without overflow, and a sum that a merge scales by a factor below the smallest normal fp32
+// number was worth less than 2^-66 of the row's.  The test costs nothing measurable (2048 x 8192 of
+// 12/2/128, scores N(0, 1): 163.6 us without it, 164.0 with), the updates 2-5% at N(0, 45^2) and
+// N(0, 80^2) (168, 172 us), where repeating a segment whose sum overflowed took 240.
+constexpr float kPfSumBound = 0x1p60f;
+
 // bf16(x) as fp32: the pair conversion with a zero low half leaves the value in place.
 __device__ __forceinline__ float rnd(float x) { return __builtin_bit_cast(float, pack_bf16x2(0.0f, x)); }
 
@@ -291,7 +300,8 @@ void prefill_kernel(AttnArgs a, int layers) {
       }
       merge_lanes<32>(m, l);
       // p = exp(s - M) / L as one exp2: 2^(s log2 e - M log2 e - log2 L) (v_log_f32 is within
-      // 1 ulp; |log2 L| <= log2 T, so p moves by ~1e-6 relative, far below its BF16 step)
+      // 1 ulp; 1 <= L < 2^67, kPfSumBound for each of two lanes and at most 64 segments, so its
+      // rounding moves p by less than 5e-6 relative, far below its BF16 step)
       if (l > 0.0f) nml = -m * kLog2e - __builtin_amdgcn_logf(l);
     }
     // the keys every row of the wavefront sees whole, in units (scalar)
@@ -299,242 +309,235 @@ void prefill_kernel(AttnArgs a, int layers) {
 #pragma unroll
     for (int off = 16; off > 0; off >>= 1) kmin = min(kmin, __shfl_xor(kmin, off));
     const bool active = rg * kPfRows + wave * 32 < a.R;  // the wavefront has rows
+    const uint64_t rows = __ballot(rv);                  // the lanes that stand for one
     const int ufull = __builtin_amdgcn_readfirstlane(kmin == INT_MAX ? 0 : (kmin + 1) >> 5);
 
     f32x16 acc[OUT ? DT : 1];
     float m_run = -INFINITY, l_run = 0.0f;  // pass 1
-    bool slow = false;                      // pass 1: every stage through the online update
-    for (;;) {
-      if constexpr (OUT) {
+    if constexpr (OUT) {
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) acc[dt] = (f32x16)0.0f;
-      }
-      for (int wlo = slo; wlo < shi; wlo += kPfIds / 4) {  // page-id windows; workgroup-uniform
-        const int nit = min(kPfIds / 4, shi - wlo);        // stages in the window
-        if (wlo > slo) stage_ids(wlo);
-        const bool bad = __builtin_amdgcn_readfirstlane(s_bad) == window;  // an invalid id in the window
-        // units of the window (32 keys): x = 0 .. 2 nit - 1, the first at key 32 * ux0
-        const int ux0 = 2 * wlo, nx = 2 * nit;
-        const uint4* vh_grp = a.vhat + (int64_t)grp * a.vh_stages * (DT * 128) + lane;
-        // The loop multiplies q.k^T one unit ahead of the scores and p.V one unit behind them:
-        // buffer s holds K of units 2s + 1, 2s + 2 and V of units 2s - 1, 2s.  Past the window's
-        // ends the nearest unit is loaded; its products are not used, or meet p = 0.
-        int id[NK / W];   // page ids of the next fetch
-        uint4 stg[CPW];   // this wavefront's chunks of the next stage
-        auto next_ids = [&](int s) {
+      for (int dt = 0; dt < DT; ++dt) acc[dt] = (f32x16)0.0f;
+    }
+    for (int wlo = slo; wlo < shi; wlo += kPfIds / 4) {  // page-id windows; workgroup-uniform
+      const int nit = min(kPfIds / 4, shi - wlo);        // stages in the window
+      if (wlo > slo) stage_ids(wlo);
+      const bool bad = __builtin_amdgcn_readfirstlane(s_bad) == window;  // an invalid id in the window
+      // units of the window (32 keys): x = 0 .. 2 nit - 1, the first at key 32 * ux0
+      const int ux0 = 2 * wlo, nx = 2 * nit;
+      const uint4* vh_grp = a.vhat + (int64_t)grp * a.vh_stages * (DT * 128) + lane;
+      // The loop multiplies q.k^T one unit ahead of the scores and p.V one unit behind them:
+      // buffer s holds K of units 2s + 1, 2s + 2 and V of units 2s - 1, 2s.  Past the window's
+      // ends the nearest unit is loaded; its products are not used, or meet p = 0.
+      int id[NK / W];   // page ids of the next fetch
+      uint4 stg[CPW];   // this wavefront's chunks of the next stage
+      auto next_ids = [&](int s) {
 #pragma unroll
-          for (int j = 0; j < NK / W; ++j) {
-            const int c = j * W + wave, x = min(max(2 * s + 1 + c / CU, 0), nx - 1);
-            id[j] = lpb[2 * x + (c % CU) / PU];
-          }
-        };
-        auto fetch1 = [&](int s, int j) {  // chunk j * W + wave of stage s
-          const int c = j * W + wave;
-          if (j < NK / W) {
-            const int64_t pg = max(__builtin_amdgcn_readfirstlane(id[j]), 0);
-            // cached, unlike the other kernels' K: every row group reads it again (2048 x 8192 of
+        for (int j = 0; j < NK / W; ++j) {
+          const int c = j * W + wave, x = min(max(2 * s + 1 + c / CU, 0), nx - 1);
+          id[j] = lpb[2 * x + (c % CU) / PU];
+        }
+      };
+      auto fetch1 = [&](int s, int j) {  // chunk j * W + wave of stage s
+        const int c = j * W + wave;
+        if (j < NK / W) {
+          const int64_t pg = max(__builtin_amdgcn_readfirstlane(id[j]), 0);
+          // cached, unlike the other kernels' K: every row group reads it again (2048 x 8192 of
           // 12/2/128 183 us with the streaming hint, 175 without)
           return *reinterpret_cast<const uint4*>(klayer + pg * kpage + (c % PU) * 512 + lane * 8);
-          }
-          const int cc = c - NK, x = min(max(2 * s - 1 + cc / CU, 0), nx - 1);
-          const int blk = min(2 * (ux0 + x) + (cc % CU) / PU, 2 * a.vh_stages - 1);
-          return vh_grp[(int64_t)blk * (DT * 64) + (cc % PU) * 64];
-        };
-        auto stash1 = [&](uint4* buf, int j) { buf[(j * W + wave) * 64 + lane] = stg[j]; };
-        auto publish = [&]() {
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-          __builtin_amdgcn_s_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-        };
-        // The wavefront's iterations: those of fully visible stages, then those that need the mask
-        // (pass 1: the first stage too, whose maximum the fast ones start from).
-        const int nfast = !active || bad || slow ? 0 : min(nit, max(0, (ufull - ux0) >> 1));
+        }
+        const int cc = c - NK, x = min(max(2 * s - 1 + cc / CU, 0), nx - 1);
+        const int blk = min(2 * (ux0 + x) + (cc % CU) / PU, 2 * a.vh_stages - 1);
+        return vh_grp[(int64_t)blk * (DT * 64) + (cc % PU) * 64];
+      };
+      auto stash1 = [&](uint4* buf, int j) { buf[(j * W + wave) * 64 + lane] = stg[j]; };
+      auto publish = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+      };
+      // The wavefront's iterations: those of fully visible stages, then those that need the mask
+      // (pass 1: the first stage too, whose maximum the fast ones start from).
+      const int nfast = !active || bad ? 0 : min(nit, max(0, (ufull - ux0) >> 1));
 
-        // One iteration is 2 units x NM steps.  A step issues one MFMA -- q.k^T of the next unit,
-        // and in pass 2 p.V of the one before in turn -- reads the LDS operand of the step kAhead
-        // later and works on 16 / NM scores of this unit.  The three do not depend on each other,
-        // and the scheduling barriers hold the order: an MFMA takes 32 cycles of the matrix unit, a
-        // score about as many of the VALU.  The first steps also write a chunk each of the next
-        // stage, whose loads went out an iteration ago, to the third buffer, and send the loads of
-        // the stage after it; the iteration's one barrier, at the end of the first unit, publishes
-        // the stage, so that the operand reads run on across iterations.
-        constexpr int NM = OUT ? KS + 2 * DT : KS, SPM = 16 / NM, kAhead = OUT ? 4 : 2;
-        constexpr int MS = (CPW + 1) & ~1;  // the steps that write and load chunks
-        static_assert(CPW <= NM / 2, "kLater operand reads lie between the chunk writes and the barrier");
-        constexpr int kLater = NM - MS < NM / 2 ? NM - MS : NM / 2;
-        static_assert(KS == 2 * DT && NM * SPM == 16, "q.k^T and p.V steps alternate");
-        uint4 *cur = ring[0], *nxt = ring[1], *third = ring[2];
-        auto operand = [&](const uint4* sb, int m) {  // step m: of unit m / NM, k step or tile i
-          const int un = m / NM, i = OUT ? (m % NM) / 2 : m % NM;
-          const char* kb = reinterpret_cast<const char*>(sb) + kofs;
-          return OUT && (m & 1) ? __builtin_bit_cast(bf16x8, sb[(NK + un * CU + i) * 64 + lane])
-                                : *reinterpret_cast<const bf16x8*>(kb + un * (CU * 1024) + i * 512);
-        };
-        bf16x8 op[kAhead];
-        f32x16 sc;        // products of the unit whose scores come next
-        uint32_t pw[8];   // p of the unit whose p.V product comes next: two MFMA operands
-        auto pop = [&](int h) {
-          return __builtin_bit_cast(bf16x8, make_uint4(pw[4 * h], pw[4 * h + 1], pw[4 * h + 2], pw[4 * h + 3]));
-        };
-        auto body = [&](int it, bool mask) {
-          next_ids(it + 2);
-          f32x16 sn = (f32x16)0.0f;
-          uint32_t pn[8];
-          float last = 0.0f, nm = OUT ? nml : -m_run * kLog2e;
-          float y[16];
+      // One iteration is 2 units x NM steps.  A step issues one MFMA -- q.k^T of the next unit,
+      // and in pass 2 p.V of the one before in turn -- reads the LDS operand of the step kAhead
+      // later and works on 16 / NM scores of this unit.  The three do not depend on each other,
+      // and the scheduling barriers hold the order: an MFMA takes 32 cycles of the matrix unit, a
+      // score about as many of the VALU.  The first steps also write a chunk each of the next
+      // stage, whose loads went out an iteration ago, to the third buffer, and send the loads of
+      // the stage after it; the iteration's one barrier, at the end of the first unit, publishes
+      // the stage, so that the operand reads run on across iterations.
+      constexpr int NM = OUT ? KS + 2 * DT : KS, SPM = 16 / NM, kAhead = OUT ? 4 : 2;
+      constexpr int MS = (CPW + 1) & ~1;  // the steps that write and load chunks
+      static_assert(CPW <= NM / 2, "kLater operand reads lie between the chunk writes and the barrier");
+      constexpr int kLater = NM - MS < NM / 2 ? NM - MS : NM / 2;
+      static_assert(KS == 2 * DT && NM * SPM == 16, "q.k^T and p.V steps alternate");
+      uint4 *cur = ring[0], *nxt = ring[1], *third = ring[2];
+      auto operand = [&](const uint4* sb, int m) {  // step m: of unit m / NM, k step or tile i
+        const int un = m / NM, i = OUT ? (m % NM) / 2 : m % NM;
+        const char* kb = reinterpret_cast<const char*>(sb) + kofs;
+        return OUT && (m & 1) ? __builtin_bit_cast(bf16x8, sb[(NK + un * CU + i) * 64 + lane])
+                              : *reinterpret_cast<const bf16x8*>(kb + un * (CU * 1024) + i * 512);
+      };
+      bf16x8 op[kAhead];
+      f32x16 sc;        // products of the unit whose scores come next
+      uint32_t pw[8];   // p of the unit whose p.V product comes next: two MFMA operands
+      auto pop = [&](int h) {
+        return __builtin_bit_cast(bf16x8, make_uint4(pw[4 * h], pw[4 * h + 1], pw[4 * h + 2], pw[4 * h + 3]));
+      };
+      auto body = [&](int it, bool mask) {
+        next_ids(it + 2);
+        f32x16 sn = (f32x16)0.0f;
+        uint32_t pn[8];
+        float last = 0.0f, nm = OUT ? nml : -m_run * kLog2e;
+        float y[16];
 #pragma unroll
-          for (int m = 0; m < 2 * NM; ++m) {
-            const int un = m / NM, mm = m % NM, i = OUT ? mm / 2 : mm;
-            if (OUT && (m & 1))
-              acc[i % DT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op[m % kAhead], pop(i / DT), acc[i % DT], 0, 0, 0);
-            else
-              sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op[m % kAhead], qop[i], mm == 0 ? (f32x16)0.0f : sn, 0, 0, 0);
-            op[m % kAhead] = m + kAhead < 2 * NM ? operand(cur, m + kAhead) : operand(nxt, m + kAhead - 2 * NM);
-            // lane (g, n), score e: key 8 (e / 4) + 4 g + e % 4 of the unit
-            int limb[2];
-            if (mask) {
+        for (int m = 0; m < 2 * NM; ++m) {
+          const int un = m / NM, mm = m % NM, i = OUT ? mm / 2 : mm;
+          if (OUT && (m & 1))
+            acc[i % DT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op[m % kAhead], pop(i / DT), acc[i % DT], 0, 0, 0);
+          else
+            sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op[m % kAhead], qop[i], mm == 0 ? (f32x16)0.0f : sn, 0, 0, 0);
+          op[m % kAhead] = m + kAhead < 2 * NM ? operand(cur, m + kAhead) : operand(nxt, m + kAhead - 2 * NM);
+          // lane (g, n), score e: key 8 (e / 4) + 4 g + e % 4 of the unit
+          int limb[2];
+          if (mask) {
 #pragma unroll
-              for (int h = 0; h < 2; ++h) limb[h] = lpb[2 * (2 * it + un) + h] >= 0 ? lim - 32 * (ux0 + 2 * it + un) - 4 * g : -1;
+            for (int h = 0; h < 2; ++h) limb[h] = lpb[2 * (2 * it + un) + h] >= 0 ? lim - 32 * (ux0 + 2 * it + un) - 4 * g : -1;
+          }
+#pragma unroll
+          for (int e = mm * SPM; e < (mm + 1) * SPM; ++e) {
+            float v = eager(sc[e]);
+            if (mask) v = 8 * (e >> 2) + (e & 3) <= limb[e >> 3] ? v : -INFINITY;
+            if (!OUT && mask) {
+              y[e] = v;
+              continue;
             }
-#pragma unroll
-            for (int e = mm * SPM; e < (mm + 1) * SPM; ++e) {
-              float v = eager(sc[e]);
-              if (mask) v = 8 * (e >> 2) + (e & 3) <= limb[e >> 3] ? v : -INFINITY;
-              if (!OUT && mask) {
-                y[e] = v;
-                continue;
-              }
-              const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(v, kExpCoef, nm));
-              if (OUT) {
-                if (e & 1)
-                  pn[e / 2] = pack_bf16x2(last, p);
-                else
-                  last = p;
-              } else {
-                y[e & 3] = e < 4 ? p : y[e & 3] + p;
-              }
-            }
-            if (m < CPW) {
-              stash1(nxt, m);
-              stg[m] = fetch1(it + 2, m);
-            }
-            if (SPM > 1 || (m & 1)) __builtin_amdgcn_sched_barrier(0);
-            if (m == MS - 1) asm volatile("" ::: "memory");
-            if (m == NM - 1) {
-              // LDS operations of a wavefront complete in order: with at most kLater outstanding, all
-              // issued after the writes (the operand reads of steps MS .. NM - 1), the writes are done
-              asm volatile("" ::: "memory");
-              __builtin_amdgcn_s_waitcnt(0xC07F | (kLater << 8));
-              __builtin_amdgcn_s_barrier();
-              asm volatile("" ::: "memory");
-              __builtin_amdgcn_sched_barrier(0);
-            }
-            if (mm == NM - 1) {
-              sc = sn;
-              if constexpr (OUT) {
-#pragma unroll
-                for (int w = 0; w < 8; ++w) pw[w] = pn[w];
-              } else {
-#pragma clang fp contract(off)
-                if (mask) {
-                  // Online (max, sum) per lane: the running sum rescaled by
-                  // exp2((m_old - m_new) log2 e), which is exactly 1 while the max stays (the one-FMA
-                  // form exp2(m_old log2 e - RN(m_new log2 e)) is off by the product's rounding on
-                  // every update, and L drifted by ~1e-5 at T = 8192: rel-L2 7e-4 against eager)
-                  float mt = -INFINITY;
-#pragma unroll
-                  for (int w = 0; w < 16; w += 2) mt = max3f(mt, y[w], y[w + 1]);
-                  mt *= kUnit;
-                  if (mt != -INFINITY) {
-                    const float mn = fmaxf(m_run, mt);
-                    const float f = __builtin_amdgcn_exp2f((m_run - mn) * kLog2e);
-                    nm = -mn * kLog2e;
-#pragma unroll
-                    for (int w = 0; w < 16; ++w) y[w] = __builtin_amdgcn_exp2f(__builtin_fmaf(y[w], kExpCoef, nm));
-#pragma unroll
-                    for (int w = 4; w < 16; ++w) y[w & 3] = y[w & 3] + y[w];
-                    l_run = l_run * f + ((y[0] + y[1]) + (y[2] + y[3]));
-                    m_run = mn;
-                  }
-                } else {
-                  l_run = l_run + ((y[0] + y[1]) + (y[2] + y[3]));
-                }
-              }
+            const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(v, kExpCoef, nm));
+            if (OUT) {
+              if (e & 1)
+                pn[e / 2] = pack_bf16x2(last, p);
+              else
+                last = p;
+            } else {
+              y[e & 3] = e < 4 ? p : y[e & 3] + p;
             }
           }
+          if (m < CPW) {
+            stash1(nxt, m);
+            stg[m] = fetch1(it + 2, m);
+          }
+          if (SPM > 1 || (m & 1)) __builtin_amdgcn_sched_barrier(0);
+          if (m == MS - 1) asm volatile("" ::: "memory");
+          if (m == NM - 1) {
+            // LDS operations of a wavefront complete in order: with at most kLater outstanding, all
+            // issued after the writes (the operand reads of steps MS .. NM - 1), the writes are done
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0xC07F | (kLater << 8));
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          if (mm == NM - 1) {
+            if constexpr (OUT) {
+#pragma unroll
+              for (int w = 0; w < 8; ++w) pw[w] = pn[w];
+            } else {
+#pragma clang fp contract(off)
+              const float add = (y[0] + y[1]) + (y[2] + y[3]);  // of the unit's exponentials
+              bool online = mask;
+              if (!mask && (__ballot(!(l_run + add < kPfSumBound)) & rows)) {  // scalar
+#pragma unroll
+                for (int w = 0; w < 16; ++w) y[w] = eager(sc[w]);
+                online = true;
+              }
+              if (online) {
+                // Online (max, sum) per lane: the running sum rescaled by
+                // exp2((m_old - m_new) log2 e), which is exactly 1 while the max stays (the one-FMA
+                // form exp2(m_old log2 e - RN(m_new log2 e)) is off by the product's rounding on
+                // every update, and L drifted by ~1e-5 at T = 8192: rel-L2 7e-4 against eager)
+                float mt = -INFINITY;
+#pragma unroll
+                for (int w = 0; w < 16; w += 2) mt = max3f(mt, y[w], y[w + 1]);
+                mt *= kUnit;
+                if (mt != -INFINITY) {
+                  const float mn = fmaxf(m_run, mt);
+                  const float f = __builtin_amdgcn_exp2f((m_run - mn) * kLog2e);
+                  nm = -mn * kLog2e;
+#pragma unroll
+                  for (int w = 0; w < 16; ++w) y[w] = __builtin_amdgcn_exp2f(__builtin_fmaf(y[w], kExpCoef, nm));
+#pragma unroll
+                  for (int w = 4; w < 16; ++w) y[w & 3] = y[w & 3] + y[w];
+                  l_run = l_run * f + ((y[0] + y[1]) + (y[2] + y[3]));
+                  m_run = mn;
+                }
+              } else {
+                l_run = l_run + add;
+              }
+            }
+            sc = sn;
+          }
+        }
+        uint4* const t = cur;
+        cur = nxt;
+        nxt = third;
+        third = t;
+      };
+
+      // stage 0 and unit 0's K (slot 1 of stage -1), loaded together
+      uint4 stg0[NK / W];
+      next_ids(-1);
+#pragma unroll
+      for (int j = 0; j < NK / W; ++j) stg0[j] = fetch1(-1, j);
+      next_ids(0);
+#pragma unroll
+      for (int j = 0; j < CPW; ++j) stg[j] = fetch1(0, j);
+      next_ids(1);
+#pragma unroll
+      for (int j = 0; j < NK / W; ++j) third[(j * W + wave) * 64 + lane] = stg0[j];
+#pragma unroll
+      for (int j = 0; j < CPW; ++j) {
+        stash1(cur, j);
+        stg[j] = fetch1(1, j);
+      }
+      publish();
+      {
+        const char* kb = reinterpret_cast<const char*>(third) + CU * 1024 + kofs;
+        sc = (f32x16)0.0f;
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk)
+          sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(kb + kk * 512), qop[kk], sc, 0, 0, 0);
+#pragma unroll
+        for (int w = 0; w < 8; ++w) pw[w] = 0;
+#pragma unroll
+        for (int m = 0; m < kAhead; ++m) op[m] = operand(cur, m);
+      }
+      int it = 0;
+      if (!OUT && active) body(it++, true);
+      for (; it < nfast; ++it) body(it, false);
+      if (active) {
+        for (; it < nit; ++it) body(it, true);
+      } else {  // a wavefront without rows loads its share
+        for (; it < nit; ++it) {
+          next_ids(it + 2);
+#pragma unroll
+          for (int j = 0; j < CPW; ++j) {
+            stash1(nxt, j);
+            stg[j] = fetch1(it + 2, j);
+          }
+          publish();
           uint4* const t = cur;
           cur = nxt;
           nxt = third;
           third = t;
-        };
-
-        // stage 0 and unit 0's K (slot 1 of stage -1), loaded together
-        uint4 stg0[NK / W];
-        next_ids(-1);
-#pragma unroll
-        for (int j = 0; j < NK / W; ++j) stg0[j] = fetch1(-1, j);
-        next_ids(0);
-#pragma unroll
-        for (int j = 0; j < CPW; ++j) stg[j] = fetch1(0, j);
-        next_ids(1);
-#pragma unroll
-        for (int j = 0; j < NK / W; ++j) third[(j * W + wave) * 64 + lane] = stg0[j];
-#pragma unroll
-        for (int j = 0; j < CPW; ++j) {
-          stash1(cur, j);
-          stg[j] = fetch1(1, j);
-        }
-        publish();
-        {
-          const char* kb = reinterpret_cast<const char*>(third) + CU * 1024 + kofs;
-          sc = (f32x16)0.0f;
-#pragma unroll
-          for (int kk = 0; kk < KS; ++kk)
-            sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(kb + kk * 512), qop[kk], sc, 0, 0, 0);
-#pragma unroll
-          for (int w = 0; w < 8; ++w) pw[w] = 0;
-#pragma unroll
-          for (int m = 0; m < kAhead; ++m) op[m] = operand(cur, m);
-        }
-        int it = 0;
-        if (!OUT && active) body(it++, true);
-        for (; it < nfast; ++it) body(it, false);
-        if (active) {
-          for (; it < nit; ++it) body(it, true);
-        } else {  // a wavefront without rows loads its share
-          for (; it < nit; ++it) {
-            next_ids(it + 2);
-#pragma unroll
-            for (int j = 0; j < CPW; ++j) {
-              stash1(nxt, j);
-              stg[j] = fetch1(it + 2, j);
-            }
-            publish();
-            uint4* const t = cur;
-            cur = nxt;
-            nxt = third;
-            third = t;
-          }
-        }
-        if constexpr (OUT) {  // the last unit's p.V
-          if (active) {
-#pragma unroll
-            for (int i = 0; i < 2 * DT; ++i)
-              acc[i % DT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(operand(cur, 2 * i + 1), pop(i / DT), acc[i % DT], 0, 0, 0);
-          }
         }
       }
-      if constexpr (OUT) {
-        break;
-      } else {
-        // The fast stages take exp(s - m) with the first stage's maximum m: a later score more
-        // than 88 above it overflows the sum (an infinite or undefined one ends here too), and
-        // the segment is done again with the online update in every stage.
-        if (slow || !__syncthreads_or(rv && !(l_run < INFINITY))) break;
-        slow = true;
-        m_run = -INFINITY;
-        l_run = 0.0f;
-        stage_ids(slo);
+      if constexpr (OUT) {  // the last unit's p.V
+        if (active) {
+#pragma unroll
+          for (int i = 0; i < 2 * DT; ++i)
+            acc[i % DT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(operand(cur, 2 * i + 1), pop(i / DT), acc[i % DT], 0, 0, 0);
+        }
       }
     }
 

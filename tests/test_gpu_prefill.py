@@ -222,8 +222,9 @@ def test_prefill_many_row_groups_and_windows(cuda_device):
 
 @pytest.mark.parametrize("h,d,s,t", [(12, 128, 300, 1500), (14, 64, 96, 900)])
 def test_prefill_late_maximum(cuda_device, h, d, s, t):
-    """Pass 1 takes its exponentials against the first stage's maximum and repeats a segment whose
-    sum overflows: scores that jump by far more than 88 in a later stage of the same segment."""
+    """Pass 1 takes its exponentials against an earlier maximum and goes through the online update
+    where a sum would leave its bound: scores that jump by far more than 88 in a later stage of the
+    same segment, so that the exponentials themselves overflow."""
     announce(f"prefill late maximum {h}/2/{d} S={s} T={t}")
     g = wl.gen(760 + d, cuda_device)
     cache = PagedKVCache(2, d, num_blocks=t // 16 + 3, device=cuda_device, seed=761, growable=False)
@@ -268,3 +269,50 @@ def test_prefill_skips_invalid_blocks(cuda_device):
         n = int((pos <= t - s + i).sum())
         want = oatt.eager_attention(q[:, :, i:i + 1].cpu(), kc.cpu()[None][:, :, pos[:n]], v_hat[:, :, pos[:n]])
         assert_close(out[:, :, i:i + 1].cpu(), want, f"row {i}")
+
+
+@pytest.mark.parametrize("where", ["halves", "segments", "low"])
+@pytest.mark.parametrize("jump", [20.0, 60.0, 82.0, 88.5])
+@pytest.mark.parametrize("h,d", [(12, 128), (14, 64)])
+def test_prefill_finite_jumps(cuda_device, h, d, jump, where):
+    """Pass 1 sums exponentials against an earlier maximum; scores that jump by less than what
+    overflows one exponential (88.7) must neither overflow the sums that are merged afterwards --
+    of a row's two lanes (keys 3 and 5 of a stage: "halves") or of its segments (one key in every
+    other stage: "segments") -- nor, 200 below zero ("low"), lose a segment whose maximum the merge
+    finds far below another's.  Every element of q is 1, so the scores are exact."""
+    announce(f"prefill finite jumps {h}/2/{d} {where} {jump}")
+    g = wl.gen(780 + d, cuda_device)
+    s, t, base = 80, 2048, -200.0 if where == "low" else 0.0
+    score = torch.full((t,), base, device=cuda_device)
+    score[(torch.arange(2, t // 64, 7, device=cuda_device)[:, None] * 64 + torch.tensor([3, 5], device=cuda_device)).flatten()
+          if where == "halves" else torch.arange(67, t, 128, device=cuda_device)] = base + jump
+    k = (score / d ** 0.5)[:, None, None].expand(t, 2, d).to(torch.bfloat16).contiguous()
+    v = torch.randn((t, 2, d), generator=g, device=cuda_device).to(torch.bfloat16)
+    q = torch.ones((1, h, s, d), dtype=torch.bfloat16, device=cuda_device)
+    cache = PagedKVCache(2, d, num_blocks=t // 16 + 3, device=cuda_device, seed=781, growable=False)
+    cache.prefill(0, k, v, [t])
+    kp, vp, vs = cache.layer(0)
+    out = ops.paged_attention(q, kp, vp, vs, cache.block_table(), cache.seq_lens_tensor(), t)
+    torch.cuda.synchronize()
+    kc, vc, sc = cache.gather(0, 0)
+    v_hat = oq.dequantize_kv_fp8(vc.cpu()[None], sc.cpu()[None], torch.bfloat16)
+    assert_close(out.cpu(), oatt.eager_attention(q.cpu(), kc.cpu()[None], v_hat), f"{where} {jump}")
+
+
+@pytest.mark.parametrize("h,d,s,t", [(12, 128, 300, 1500), (14, 64, 777, 3000)])
+def test_prefill_wide_scores(cuda_device, h, d, s, t):
+    """Scores of N(0, 45^2): a row's maximum rises by far more than an exponential's range, in
+    steps.  Whole numbers in q and K, so that both sides round the same products."""
+    announce(f"prefill wide scores {h}/2/{d} S={s} T={t}")
+    g = wl.gen(790 + d, cuda_device)
+    k = torch.randint(-11, 12, (t, 2, d), generator=g, device=cuda_device).to(torch.bfloat16)
+    v = torch.randn((t, 2, d), generator=g, device=cuda_device).to(torch.bfloat16)
+    q = torch.randint(-11, 12, (1, h, s, d), generator=g, device=cuda_device).to(torch.bfloat16)
+    cache = PagedKVCache(2, d, num_blocks=t // 16 + 3, device=cuda_device, seed=791, growable=False)
+    cache.prefill(0, k, v, [t])
+    kp, vp, vs = cache.layer(0)
+    out = ops.paged_attention(q, kp, vp, vs, cache.block_table(), cache.seq_lens_tensor(), t)
+    torch.cuda.synchronize()
+    kc, vc, sc = cache.gather(0, 0)
+    v_hat = oq.dequantize_kv_fp8(vc.cpu()[None], sc.cpu()[None], torch.bfloat16)
+    assert_close(out.cpu(), oatt.eager_attention(q.cpu(), kc.cpu()[None], v_hat), "wide scores")
