@@ -583,7 +583,7 @@ void prefill_kernel(AttnArgs a, int layers) {
     // tile 64 lanes x 16 bytes (lane (g, m): dimension 32 dt + m, tokens 4g..4g+3 and
     // 8+4g..8+4g+3).  Codes and scales of tokens that are not in the sequence (past T, invalid or
     // absent blocks) become 0, so that no NaN pattern of an unwritten slot reaches the MFMA; up
-    // to the end of the last stage every block is written.
+    // to the end of the last stage every block is written, an empty sequence's one stage too.
     typedef float f32x2 __attribute__((ext_vector_type(2)));
     const int nbmax = 2 * a.vh_stages;
     const int64_t items = (int64_t)LK * a.B * nbmax;
@@ -591,7 +591,7 @@ void prefill_kernel(AttnArgs a, int layers) {
       const int z = (int)(i / nbmax), blk = (int)(i - (int64_t)z * nbmax);
       const int zb = z / a.KV, kvh = z - zb * a.KV, layer = zb / a.B, b = zb - layer * a.B;
       const int T = seq_len_of(a, b), nbk = (T + kBlock - 1) / kBlock;
-      if (blk >= ((nbk + 3) & ~3)) continue;
+      if (blk >= max((nbk + 3) & ~3, kPfStage / kBlock)) continue;
       int pb = blk < nbk ? a.block_table[(int64_t)b * a.max_blocks + blk] : -1;
       if (pb >= a.num_blocks) pb = -1;
       const int64_t pg = max(pb, 0);

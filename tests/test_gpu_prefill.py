@@ -19,6 +19,7 @@ from conftest import announce
 from helpers import assert_close
 from oracle import attention as oatt
 from oracle import quant as oq
+from specdec_amd import _native
 from specdec_amd import workloads as wl
 from specdec_amd.engine.paged_cache import PagedKVCache
 from specdec_amd.kernels import ops
@@ -316,3 +317,32 @@ def test_prefill_wide_scores(cuda_device, h, d, s, t):
     kc, vc, sc = cache.gather(0, 0)
     v_hat = oq.dequantize_kv_fp8(vc.cpu()[None], sc.cpu()[None], torch.bfloat16)
     assert_close(out.cpu(), oatt.eager_attention(q.cpu(), kc.cpu()[None], v_hat), "wide scores")
+
+
+@pytest.mark.parametrize("h,d,s,lens", [(12, 128, 80, [700, 0, 300]), (14, 64, 96, [0, 500]),
+                                        (12, 128, 11, [300] * 64 + [0] * 3 + [300] * 63)])
+def test_prefill_empty_sequence(cuda_device, h, d, s, lens):
+    """A sequence without tokens in a prefill batch gives zeros whatever the workspace held (NaN bits
+    here), in ranges of stages and (130 sequences) in whole row groups; the others are as without
+    it.  The sequences share one sequence's pages."""
+    announce(f"prefill with empty sequences {h}/2/{d} S={s} batch {len(lens)}")
+    g = wl.gen(800 + d + s, cuda_device)
+    t, b = max(lens), len(lens)
+    cache = PagedKVCache(2, d, num_blocks=t // 16 + 3, device=cuda_device, seed=801, growable=False)
+    cache.prefill(0, torch.randn((t, 2, d), generator=g, device=cuda_device).to(torch.bfloat16),
+                  torch.randn((t, 2, d), generator=g, device=cuda_device).to(torch.bfloat16), [t])
+    q = torch.randn((b, h, s, d), generator=g, device=cuda_device).to(torch.bfloat16)
+    kp, vp, vs = cache.layer(0)
+    ws = ops.new_workspace(cuda_device, ops.attention_workspace_bytes(1, b, h, 2, s, d, t))
+    ws[_native.SYNC_BYTES:] = 0xFF
+    out = ops.paged_attention(q, kp, vp, vs, cache.block_table().expand(b, -1).contiguous(),
+                              torch.tensor(lens, dtype=torch.int32, device=cuda_device), t, workspace_tensor=ws)
+    torch.cuda.synchronize()
+    kc, vc, sc = cache.gather(0, 0)
+    v_hat = oq.dequantize_kv_fp8(vc.cpu()[None], sc.cpu()[None], torch.bfloat16)
+    for i, n in enumerate(lens):
+        if n == 0:
+            assert not out[i].any(), f"sequence {i} is empty"
+        elif i < 3 or i == b - 1:
+            want = oatt.eager_attention(q[i:i + 1].cpu(), kc.cpu()[None][:, :, :n], v_hat[:, :, :n])
+            assert_close(out[i:i + 1].cpu(), want, f"sequence {i} of {n}")
