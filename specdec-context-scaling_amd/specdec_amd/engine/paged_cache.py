@@ -98,6 +98,9 @@ class PagedKVCache:
         self.lengths: list[int] = [0] * batch
         self._bt = None
         self._tiles = None  # (lengths, stream, device tile table) of the last prefill
+        # tile tables that recorded graphs read, by lengths (which alone decide a table's contents):
+        # kept alive as long as the pool, one for each set of lengths recorded
+        self._recorded: dict[tuple, torch.Tensor] = {}
         self._ws = None     # attention workspace owned by the pool
         # replaced workspaces, kept alive for graphs that recorded them; each replacement is at
         # least twice the size of the one before, so they hold at most the current one's bytes
@@ -306,9 +309,10 @@ class PagedKVCache:
             if n > len(self.blocks[b]) * BLOCK:
                 self.reserve(b, n)
         on_device = self.device.type == "cuda"
-        key = (tuple(lengths), ops._stream(self.device) if on_device else 0)
+        key = (tuple(lengths), ops._stream(self.k_pages.device) if on_device else 0)
         stale = self._tiles is None or self._tiles[:2] != key
-        if on_device and (slots is None or stale) and not _recording(self.device):
+        recording = on_device and _recording(self.device)
+        if on_device and (slots is None or stale) and not recording:
             fresh, table = self._varlen(lengths)
             slots = fresh if slots is None else slots
             self._tiles = (*key, table)
@@ -318,11 +322,13 @@ class PagedKVCache:
             if stale:
                 table = torch.tensor(ops.varlen_tile_starts(list(lengths)), dtype=torch.int32).to(self.device)
                 self._tiles = (*key, table)
+        table = self._recorded.setdefault(key[0], self._tiles[2]) if recording else self._tiles[2]
         pages = self._layer_pointers(layer, v_new.device) if on_device else None
-        if not ops.quant_append_pages(v_new, k_new, slots, pages, self._tiles[2], self.kv_heads, self.head_dim, self.scale_mode):
+        if not ops.quant_append_pages(v_new, k_new, slots, pages, table, self.kv_heads, self.head_dim, self.scale_mode,
+                                      key[1]):
             kp, vp, vs = self.layer(layer)
             ops.quant_append(v_new, slots, kp, vp, vs, k_new, scale_mode=self.scale_mode,
-                             tile_starts=self._tiles[2])
+                             tile_starts=table)
         self.lengths[:] = lengths
         return slots
 

@@ -468,9 +468,10 @@ def append_attend_pages(q, k_new, v_new, pages, block_table, max_seq_len, B, S, 
     return out
 
 
-def quant_append_pages(v_new, k_new, slots, pages, tile_starts, KV, D, scale_mode) -> bool:
+def quant_append_pages(v_new, k_new, slots, pages, tile_starts, KV, D, scale_mode, stream) -> bool:
     """quant_append of one layer of a pool whose page addresses the caller has; False (nothing
-    done) when an argument is not the plain tensor that the call's fixed arguments stand for."""
+    done) when an argument is not the plain tensor that the call's fixed arguments stand for.
+    `stream` is the current one of v_new's device (where `pages` is not None, the pool's)."""
     if pages is None or not isinstance(v_new, torch.Tensor) or v_new.dim() != 3 or scale_mode not in _SCALE_MODES:
         return False
     dev, n = v_new.device, v_new.shape[0]
@@ -480,7 +481,7 @@ def quant_append_pages(v_new, k_new, slots, pages, tile_starts, KV, D, scale_mod
     kp, vp, sp, nb = pages
     st = _native.load().sdv_quant_append_tiles(
         v_new.data_ptr(), k_new.data_ptr(), slots.data_ptr(), n, KV, D, D, 1, 0, kp, vp, sp, nb, 0, 0, 0,
-        _SCALE_MODES[scale_mode], tile_starts.data_ptr(), tile_starts.shape[0] - 1, _stream(dev))
+        _SCALE_MODES[scale_mode], tile_starts.data_ptr(), tile_starts.shape[0] - 1, stream)
     if st:
         _native.check(st, "sdv_quant_append_tiles")
     return True

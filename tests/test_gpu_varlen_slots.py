@@ -65,3 +65,50 @@ def test_varlen_slots_refuse_unreserved_positions(cuda_device):
         cache.varlen_slots([49])
     with pytest.raises(RuntimeError):
         ops.varlen_slots(cache.block_table(), [1, 2, 3])
+
+
+def _replay_test(cuda_device, warm, record):
+    """Record prefill with the slots of a warm-up on stream `warm` (capture stream `record`), then
+    replay it with new K and V between eager prefills that replace the pool's tables, with whatever
+    those freed overwritten; every replay gives the pages of the same call run eagerly."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(11)
+    lengths, others = [37, 80, 5], ([80, 5, 37], [37, 80, 5], [1, 1, 1])
+    k = torch.zeros((sum(lengths), 2, 64), dtype=torch.bfloat16, device="cuda")
+    v = torch.zeros_like(k)
+    cache = PagedKVCache(2, 64, batch=3, num_blocks=18, device=cuda_device, seed=12, growable=False)
+    for b in range(3):
+        cache.reserve(b, 80)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(warm):
+        slots = cache.prefill(0, k, v, lengths)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=record):
+        cache.prefill(0, k, v, lengths, slots)
+    for i, other in enumerate(others):
+        with torch.cuda.stream(torch.cuda.Stream() if i % 2 else record):
+            cache.prefill(0, *(2 * [torch.randn((sum(other), 2, 64), generator=g, device="cuda").to(torch.bfloat16)]), other)
+        torch.cuda.synchronize()
+        junk = [torch.full((n,), 3, dtype=torch.int32, device="cuda") for n in (8, 16, 64, 128, 256) for _ in range(8)]
+        k.copy_(torch.randn(k.shape, generator=g, device="cuda"))
+        v.copy_(torch.randn(k.shape, generator=g, device="cuda"))
+        for x in (cache.k_pages, cache.v_pages, cache.v_scales):
+            x.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        ref = PagedKVCache(2, 64, batch=3, num_blocks=18, device=cuda_device, seed=12, growable=False)
+        for x in (ref.k_pages, ref.v_pages, ref.v_scales):
+            x.zero_()
+        ops.quant_append(v, slots, *ref.layer(0), k)
+        torch.cuda.synchronize()
+        for x, y in zip(cache.layer(0), ref.layer(0)):
+            assert torch.equal(x, y), f"replay {i}"
+        del junk
+
+
+def test_recorded_prefill_keeps_its_table(cuda_device):
+    """A table that a graph reads outlives the prefills that replace it."""
+    announce("recorded prefill, table kept")
+    side = torch.cuda.Stream()
+    _replay_test(cuda_device, side, side)
