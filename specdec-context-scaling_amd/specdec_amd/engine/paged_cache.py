@@ -276,7 +276,8 @@ class PagedKVCache:
     def varlen_slots(self, lengths: list[int]) -> torch.Tensor:
         """int32 (sum(lengths),) slots of positions 0..lengths[b]-1 of each sequence in turn (on a
         device, written by a kernel on the current stream)."""
-        if self.device.type == "cuda" and not _recording(self.device):
+        if self.device.type == "cuda":
+            _no_recording(self.device, "slots would be built")
             return self._varlen(lengths, tiles=False)[0]
         out = []
         for b, n in enumerate(lengths):
@@ -301,7 +302,8 @@ class PagedKVCache:
         lengths become ``lengths``.  Returns the slot mapping so that later layers can pass it
         (written by a kernel on the current stream, like any result).  The launch takes a tile
         table that starts a tile at every sequence's first row (built with the slots, once per set
-        of lengths and stream), so whole page blocks are written with 16-byte stores.
+        of lengths and stream), so whole page blocks are written with 16-byte stores.  A recorded
+        call takes the table of an earlier call with the same lengths, and needs its slots.
         """
         if len(lengths) != self.batch:
             raise ValueError(f"{len(lengths)} lengths for a batch of {self.batch}")
@@ -311,18 +313,26 @@ class PagedKVCache:
         on_device = self.device.type == "cuda"
         key = (tuple(lengths), ops._stream(self.k_pages.device) if on_device else 0)
         stale = self._tiles is None or self._tiles[:2] != key
-        recording = on_device and _recording(self.device)
-        if on_device and (slots is None or stale) and not recording:
-            fresh, table = self._varlen(lengths)
-            slots = fresh if slots is None else slots
-            self._tiles = (*key, table)
+        if on_device and _recording(self.device):
+            # the table of an earlier call with these lengths, whichever stream it ran on (the
+            # capture stream is usually another)
+            warm = self._tiles is not None and self._tiles[0] == key[0]
+            if slots is None or not (warm or key[0] in self._recorded):
+                _no_recording(self.device, "prefill would build its tables (call it with these lengths before, and pass the "
+                                           "slots that it returns)")
+            table = self._recorded.setdefault(key[0], self._tiles[2])
+        elif on_device:
+            if slots is None or stale:
+                fresh, table = self._varlen(lengths)
+                slots = fresh if slots is None else slots
+                self._tiles = (*key, table)
+            table = self._tiles[2]
         else:
             if slots is None:
                 slots = self.varlen_slots(lengths)
             if stale:
-                table = torch.tensor(ops.varlen_tile_starts(list(lengths)), dtype=torch.int32).to(self.device)
-                self._tiles = (*key, table)
-        table = self._recorded.setdefault(key[0], self._tiles[2]) if recording else self._tiles[2]
+                self._tiles = (*key, torch.tensor(ops.varlen_tile_starts(list(lengths)), dtype=torch.int32))
+            table = self._tiles[2]
         pages = self._layer_pointers(layer, v_new.device) if on_device else None
         if not ops.quant_append_pages(v_new, k_new, slots, pages, table, self.kv_heads, self.head_dim, self.scale_mode,
                                       key[1]):

@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from conftest import announce
+from specdec_amd import SdvError
 from specdec_amd.engine.paged_cache import PagedKVCache
 from specdec_amd.kernels import ops
 
@@ -112,3 +113,33 @@ def test_recorded_prefill_keeps_its_table(cuda_device):
     announce("recorded prefill, table kept")
     side = torch.cuda.Stream()
     _replay_test(cuda_device, side, side)
+
+
+def test_prefill_records_on_another_stream(cuda_device):
+    """The warm-up's table serves a recording on the capture stream, as torch.cuda.graph makes one;
+    lengths not called before, and a recording without slots, are refused before anything is copied,
+    and the recording goes on."""
+    announce("recorded prefill, capture stream")
+    _replay_test(cuda_device, torch.cuda.Stream(), torch.cuda.Stream())
+    _replay_test(cuda_device, torch.cuda.current_stream(), torch.cuda.Stream())
+    k = torch.randn((40, 2, 64), device="cuda").to(torch.bfloat16)
+    cache = PagedKVCache(2, 64, batch=1, num_blocks=4, device=cuda_device)
+    slots = cache.prefill(0, k, k, [40])
+    torch.cuda.synchronize()
+    want = [x.clone() for x in cache.layer(0)]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        with pytest.raises(SdvError, match="recorded"):
+            cache.prefill(0, k, k, [40])
+        with pytest.raises(SdvError, match="recorded"):
+            cache.prefill(0, k[:39], k[:39], [39], slots[:39])
+        with pytest.raises(SdvError, match="recorded"):
+            cache.varlen_slots([40])
+        cache.prefill(0, k, k, [40], slots)
+    for _ in range(3):
+        for x in cache.layer(0):
+            x.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for x, y in zip(cache.layer(0), want):
+            assert torch.equal(x[cache.blocks[0][:2]], y[cache.blocks[0][:2]])   # whole blocks
