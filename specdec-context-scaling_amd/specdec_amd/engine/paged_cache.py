@@ -98,6 +98,9 @@ class PagedKVCache:
         self.lengths: list[int] = [0] * batch
         self._bt = None
         self._tiles = None  # (lengths, stream, device tile table) of the last prefill
+        # stream of the last kernel that wrote slots or tiles, and, once a second stream has been
+        # seen, an event after it (recording one costs 8 us of host time)
+        self._written, self._event = None, None
         # tile tables that recorded graphs read, by lengths (which alone decide a table's contents):
         # kept alive as long as the pool, one for each set of lengths recorded
         self._recorded: dict[tuple, torch.Tensor] = {}
@@ -292,18 +295,35 @@ class PagedKVCache:
         for b, n in enumerate(lengths):
             if n < 0 or -(-n // BLOCK) > len(self.blocks[b]):
                 raise IndexError(f"sequence {b} has {len(self.blocks[b])} blocks, {n} positions asked for")
-        return ops.varlen_slots(self.block_table(), lengths, tiles=tiles)
+        got = ops.varlen_slots(self.block_table(), lengths, tiles=tiles)
+        stream = ops._stream(self.k_pages.device)
+        if self._written not in (None, stream):
+            self._after_tables()  # so that the event stands for those written before as well
+        self._written = stream
+        if self._event is not None:
+            self._event.record(torch.cuda.current_stream(self.k_pages.device))
+        return got
+
+    def _after_tables(self) -> None:
+        """The current stream goes on after the slots and tiles written so far on another one: a
+        prefill may be given slots that were made there.  The first time, the host waits."""
+        if self._event is None:
+            torch.cuda.synchronize(self.k_pages.device)
+            self._event = torch.cuda.Event()
+            self._event.record(torch.cuda.current_stream(self.k_pages.device))
+        torch.cuda.current_stream(self.k_pages.device).wait_event(self._event)
 
     def prefill(self, layer: int, k_new: torch.Tensor, v_new: torch.Tensor, lengths: list[int],
                 slots: torch.Tensor | None = None) -> torch.Tensor:
         """Write whole prompts of different lengths into one layer (one kernel 1 launch).
 
         k_new/v_new BF16 (sum(lengths), KV, D), sequence after sequence (the varlen layout);
-        lengths become ``lengths``.  Returns the slot mapping so that later layers can pass it
-        (written by a kernel on the current stream, like any result).  The launch takes a tile
-        table that starts a tile at every sequence's first row (built with the slots, once per set
-        of lengths and stream), so whole page blocks are written with 16-byte stores.  A recorded
-        call takes the table of an earlier call with the same lengths, and needs its slots.
+        lengths become ``lengths``.  Returns the slot mapping so that later layers can pass it, on
+        any stream (a kernel on the current one writes it; prefill on another waits for that).  The
+        launch takes a tile table that starts a tile at every sequence's first row (built with the
+        slots, once per set of lengths and stream), so whole page blocks are written with 16-byte
+        stores.  A recorded call takes the table of an earlier call with the same lengths, and needs
+        its slots; replays come after that call, like any use of its pages.
         """
         if len(lengths) != self.batch:
             raise ValueError(f"{len(lengths)} lengths for a batch of {self.batch}")
@@ -313,7 +333,7 @@ class PagedKVCache:
         on_device = self.device.type == "cuda"
         key = (tuple(lengths), ops._stream(self.k_pages.device) if on_device else 0)
         stale = self._tiles is None or self._tiles[:2] != key
-        if on_device and _recording(self.device):
+        if on_device and torch.cuda.is_current_stream_capturing():
             # the table of an earlier call with these lengths, whichever stream it ran on (the
             # capture stream is usually another)
             warm = self._tiles is not None and self._tiles[0] == key[0]
@@ -326,6 +346,8 @@ class PagedKVCache:
                 fresh, table = self._varlen(lengths)
                 slots = fresh if slots is None else slots
                 self._tiles = (*key, table)
+            elif self._written != key[1]:
+                self._after_tables()
             table = self._tiles[2]
         else:
             if slots is None:

@@ -143,3 +143,40 @@ def test_prefill_records_on_another_stream(cuda_device):
         torch.cuda.synchronize()
         for x, y in zip(cache.layer(0), want):
             assert torch.equal(x[cache.blocks[0][:2]], y[cache.blocks[0][:2]])   # whole blocks
+
+
+def test_prefill_takes_slots_of_a_busy_stream(cuda_device):
+    """Slots made on one stream and passed to a later layer's prefill on another: the second stream
+    waits for the kernel that writes them, also where its own table need not be built again."""
+    announce("prefill, slots of a busy stream")
+    lengths = [300, 41]
+    k = torch.randn((sum(lengths), 2, 64), device="cuda").to(torch.bfloat16)
+    cache, ref = (PagedKVCache(2, 64, num_layers=3, batch=2, num_blocks=24, device=cuda_device, seed=6) for _ in range(2))
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    x = torch.randn((4096, 4096), device="cuda").to(torch.bfloat16)
+    for c in (cache, ref):
+        for i, n in enumerate(lengths):
+            c.reserve(i, n)
+        c.block_table()
+    torch.cuda.synchronize()
+
+    def busy():
+        for _ in range(200):
+            x @ x
+
+    with torch.cuda.stream(a):
+        busy()
+        slots = cache.prefill(0, k, k, lengths)
+    with torch.cuda.stream(b):
+        cache.prefill(1, k, k, lengths, slots)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(a):
+        busy()
+        again = cache.varlen_slots(lengths)
+    with torch.cuda.stream(b):
+        cache.prefill(2, k, k, lengths, again)
+    torch.cuda.synchronize()
+    for layer in range(3):
+        ops.quant_append(k, _host(ref, lengths)[0].cuda(), *ref.layer(layer), k)
+    torch.cuda.synchronize()
+    assert torch.equal(cache.k_pages, ref.k_pages) and torch.equal(cache.v_pages, ref.v_pages)
