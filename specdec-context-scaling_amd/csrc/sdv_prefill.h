@@ -87,12 +87,13 @@ __device__ __forceinline__ int wave_scan(int v) {
 }
 
 // Bound of pass 1's sums of exponentials in the fully visible stages, whose exponents are taken
-// against an earlier maximum: a unit that would bring a lane's sum to this much goes through the
+// against an earlier maximum: a stage that would bring a lane's sum to this much goes through the
 // online update instead.  The two lanes of a row and its segments (at most 64) can then be added
 // without overflow, and a sum that a merge scales by a factor below the smallest normal fp32
-// number was worth less than 2^-66 of the row's.  The test costs nothing measurable (2048 x 8192 of
-// 12/2/128, scores N(0, 1): 163.6 us without it, 164.0 with), the updates 2-5% at N(0, 45^2) and
-// N(0, 80^2) (168, 172 us), where repeating a segment whose sum overflowed took 240.
+// number was worth less than 2^-66 of the row's.  Tested once per stage, for which the first unit's
+// products are kept: a test per unit cost pass 1 of head_dim 64 6% (2048 x 16000, both passes 217 us
+// without a bound, 225 with a test per unit, 216 with one per stage).  The updates cost 2-5% at scores
+// of N(0, 45^2) and N(0, 80^2), where repeating a segment whose sum overflowed cost 40%.
 constexpr float kPfSumBound = 0x1p60f;
 
 // bf16(x) as fp32: the pair conversion with a zero low half leaves the value in place.
@@ -385,12 +386,35 @@ void prefill_kernel(AttnArgs a, int layers) {
       auto pop = [&](int h) {
         return __builtin_bit_cast(bf16x8, make_uint4(pw[4 * h], pw[4 * h + 1], pw[4 * h + 2], pw[4 * h + 3]));
       };
+      // Pass 1's online (max, sum) per lane of a unit's scores y: the running sum rescaled by
+      // exp2((m_old - m_new) log2 e), which is exactly 1 while the max stays (the one-FMA form
+      // exp2(m_old log2 e - RN(m_new log2 e)) is off by the product's rounding on every update, and
+      // L drifted by ~1e-5 at T = 8192: rel-L2 7e-4 against eager).
+      auto online = [&](float (&y)[16]) {
+#pragma clang fp contract(off)
+        float mt = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < 16; w += 2) mt = max3f(mt, y[w], y[w + 1]);
+        mt *= kUnit;
+        if (mt != -INFINITY) {
+          const float mn = fmaxf(m_run, mt);
+          const float f = __builtin_amdgcn_exp2f((m_run - mn) * kLog2e), nm = -mn * kLog2e;
+#pragma unroll
+          for (int w = 0; w < 16; ++w) y[w] = __builtin_amdgcn_exp2f(__builtin_fmaf(y[w], kExpCoef, nm));
+#pragma unroll
+          for (int w = 4; w < 16; ++w) y[w & 3] = y[w & 3] + y[w];
+          l_run = l_run * f + ((y[0] + y[1]) + (y[2] + y[3]));
+          m_run = mn;
+        }
+      };
       auto body = [&](int it, bool mask) {
         next_ids(it + 2);
         f32x16 sn = (f32x16)0.0f;
         uint32_t pn[8];
-        float last = 0.0f, nm = OUT ? nml : -m_run * kLog2e;
+        float last = 0.0f, l_next = 0.0f;
+        const float nm = OUT ? nml : -m_run * kLog2e;
         float y[16];
+        f32x16 first;  // pass 1: the first unit's products, should the sum leave its bound
 #pragma unroll
         for (int m = 0; m < 2 * NM; ++m) {
           const int un = m / NM, mm = m % NM, i = OUT ? mm / 2 : mm;
@@ -444,35 +468,23 @@ void prefill_kernel(AttnArgs a, int layers) {
               for (int w = 0; w < 8; ++w) pw[w] = pn[w];
             } else {
 #pragma clang fp contract(off)
-              const float add = (y[0] + y[1]) + (y[2] + y[3]);  // of the unit's exponentials
-              bool online = mask;
-              if (!mask && (__ballot(!(l_run + add < kPfSumBound)) & rows)) {  // scalar
-#pragma unroll
-                for (int w = 0; w < 16; ++w) y[w] = eager(sc[w]);
-                online = true;
-              }
-              if (online) {
-                // Online (max, sum) per lane: the running sum rescaled by
-                // exp2((m_old - m_new) log2 e), which is exactly 1 while the max stays (the one-FMA
-                // form exp2(m_old log2 e - RN(m_new log2 e)) is off by the product's rounding on
-                // every update, and L drifted by ~1e-5 at T = 8192: rel-L2 7e-4 against eager)
-                float mt = -INFINITY;
-#pragma unroll
-                for (int w = 0; w < 16; w += 2) mt = max3f(mt, y[w], y[w + 1]);
-                mt *= kUnit;
-                if (mt != -INFINITY) {
-                  const float mn = fmaxf(m_run, mt);
-                  const float f = __builtin_amdgcn_exp2f((m_run - mn) * kLog2e);
-                  nm = -mn * kLog2e;
-#pragma unroll
-                  for (int w = 0; w < 16; ++w) y[w] = __builtin_amdgcn_exp2f(__builtin_fmaf(y[w], kExpCoef, nm));
-#pragma unroll
-                  for (int w = 4; w < 16; ++w) y[w & 3] = y[w & 3] + y[w];
-                  l_run = l_run * f + ((y[0] + y[1]) + (y[2] + y[3]));
-                  m_run = mn;
-                }
+              if (mask) {
+                online(y);
               } else {
-                l_run = l_run + add;
+                const float sum = (un == 0 ? l_run : l_next) + ((y[0] + y[1]) + (y[2] + y[3]));
+                if (un == 0) {
+                  l_next = sum;
+                  first = sc;
+                } else if (__ballot(!(sum < kPfSumBound)) & rows) {  // scalar
+#pragma unroll
+                  for (int w = 0; w < 16; ++w) y[w] = eager(first[w]);
+                  online(y);
+#pragma unroll
+                  for (int w = 0; w < 16; ++w) y[w] = eager(sc[w]);
+                  online(y);
+                } else {
+                  l_run = sum;
+                }
               }
             }
             sc = sn;
