@@ -2013,6 +2013,7 @@ struct Plan {
   int tpad;                                       // group_kernel: scratch row length (tokens)
   int pf_nrg, pf_w1, pf_w2, pf_min1, pf_min2;     // prefill: see AttnArgs
   int pf_split, pf_slots, pf_dense;
+  bool pf_short;                                  // prefill: short contexts, row groups of 128 rows
   size_t off_vhat;                                // prefill: dequantized V (pass 1 -> pass 2)
   int vh_stages;                                  // prefill: two-block stages per group
   size_t total;                                   // bytes for every layout the call may take
@@ -2056,10 +2057,13 @@ static void plan_prefill(int64_t groups, int R, int S, int G, int D, int T, Plan
   p->off_vhat = p->off_partial + slots;
   p->total = p->off_vhat + (size_t)groups * p->vh_stages * (D / 16) * 1024;
 
+  p->pf_nrg = (R + kPfShortRows - 1) / kPfShortRows;
+  p->pf_short = pf_stages(p->pf_nrg - 1, kPfShortRows, S, G, T) <= pf_short_stages(D, groups * p->pf_nrg);
+  if (p->pf_short) return;
   p->pf_nrg = (R + kPfRows - 1) / kPfRows;
   const int64_t nrg = groups * p->pf_nrg;  // row groups of the call
   int64_t stages = 0;
-  for (int i = 0; i < p->pf_nrg; ++i) stages += kPfSegStages + pf_stages(i, S, G, T);
+  for (int i = 0; i < p->pf_nrg; ++i) stages += kPfSegStages + pf_stages(i, kPfRows, S, G, T);
   const int64_t U = stages * groups;
   const int64_t slot_b = (int64_t)kPfRows * D * 4;
   p->pf_slots = (int)(slots / slot_b);
@@ -2073,7 +2077,7 @@ static void plan_prefill(int64_t groups, int R, int S, int G, int D, int T, Plan
   p->pf_dense = w2 + nrg <= have;
   // pass 1: the ranges that cut a row group of ns stages, at most (ns - 2) / per + 2, fit its
   // statistics
-  const int ns = pf_stages(p->pf_nrg - 1, S, G, T);
+  const int ns = pf_stages(p->pf_nrg - 1, kPfRows, S, G, T);
   if (p->pf_split >= 2) {
     p->pf_w1 = (int)std::min(cap, (U + kPfMinStages - 1) / kPfMinStages);
     p->pf_min1 = std::max(p->pf_min1, (ns - 1 + p->pf_split - 2) / (p->pf_split - 1));
@@ -2118,6 +2122,7 @@ static bool make_plan(int L, int B, int H, int KV, int S, int D, int max_seq_len
   p->tpad = 0;
   p->pf_nrg = p->pf_w1 = p->pf_w2 = p->pf_min1 = p->pf_min2 = 0;
   p->pf_split = p->pf_slots = p->pf_dense = 0;
+  p->pf_short = false;
   p->off_vhat = 0;
   p->vh_stages = 0;
   if (p->n_row_groups > 1) {  // prefill kernels
@@ -2357,10 +2362,20 @@ static bool launch_all(const AttnArgs& a, const Plan& p, int zdim, hipStream_t s
     if (a.app_v) return false;
     const int layers = zdim / a.B;
     const unsigned whole = (unsigned)(p.groups * p.pf_nrg);
+    if (p.pf_short) {
+      const int64_t blocks = p.groups * p.vh_stages * 2;
+      const unsigned dequant = (unsigned)std::min<int64_t>(kPfShortVWorkgroups, (blocks + kPfShortWaves - 1) / kPfShortWaves);
+      const dim3 threads(64 * kPfShortWaves);
+      if (phases & SDV_PHASE_QK)
+        hipLaunchKernelGGL((prefill_kernel<D, false, kPfShortWaves>), dim3(whole + dequant), threads, 0, st, a, layers);
+      if (phases & SDV_PHASE_PV)
+        hipLaunchKernelGGL((prefill_kernel<D, true, kPfShortWaves>), dim3(whole), threads, 0, st, a, layers);
+      return true;
+    }
     if (phases & SDV_PHASE_QK)
-      hipLaunchKernelGGL((prefill_kernel<D, false>), dim3(p.pf_w1 ? p.pf_w1 : whole), dim3(64 * kPfWaves), 0, st, a, layers);
+      hipLaunchKernelGGL((prefill_kernel<D, false, kPfWaves>), dim3(p.pf_w1 ? p.pf_w1 : whole), dim3(64 * kPfWaves), 0, st, a, layers);
     if (phases & SDV_PHASE_PV)
-      hipLaunchKernelGGL((prefill_kernel<D, true>), dim3(p.pf_w2 ? p.pf_w2 : whole), dim3(64 * kPfWaves), 0, st, a, layers);
+      hipLaunchKernelGGL((prefill_kernel<D, true, kPfWaves>), dim3(p.pf_w2 ? p.pf_w2 : whole), dim3(64 * kPfWaves), 0, st, a, layers);
     if ((phases & SDV_PHASE_REDUCE) && p.pf_w2)
       hipLaunchKernelGGL(prefill_reduce_kernel<D>, dim3(whole * kPfWaves), dim3(256), 0, st, a);
     return true;

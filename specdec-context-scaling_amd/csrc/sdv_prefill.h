@@ -27,6 +27,12 @@
 // per workgroup instead leave the longest part to set the end: 2048 x 8192 has 96 row groups of
 // 97 to 128 stages, 42 stages per CU in equal ranges and 64 in parts of two.
 //
+// Short contexts (kPfShortStages) hold too few stages to share: what they cost is starts, merges and
+// launches.  There a workgroup of four wavefronts takes a whole row group of 128 rows, workgroups
+// of their own dequantize V beside pass 1, and no parts are left to sum.  80 x 80 of 12/2/128 28.3 ->
+// 16.0 us, 300 x 300 32.8 -> 23.1, 28 layers of 512 x 512 95 -> 78; 14/2/64 21.8 -> 12.8, 25.2 -> 16.7,
+// 70 -> 53.
+//
 // What bounds it: both passes keep the VALU and the matrix cores busy together.  A score costs
 // about 29 VALU cycles per lane in either pass (two roundings, a multiply, an FMA, v_exp_f32 at
 // half rate, and a sum or half a conversion), an MFMA 32 cycles per 16 scores of a lane; per
@@ -46,8 +52,11 @@ namespace sdv {
 
 constexpr int kPfWaves = 8;                    // wavefronts per workgroup
 constexpr int kPfRows = 32 * kPfWaves;         // rows of a row group
+constexpr int kPfShortWaves = 4;               // the same where the contexts are short
+constexpr int kPfShortRows = 32 * kPfShortWaves;
 constexpr int kPfStage = 64;                   // keys per stage: two units of 32
 constexpr int kPfIds = 2048;                   // page ids staged in LDS at a time (a multiple of 4)
+constexpr int kPfShortIds = 256;
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // One workgroup per CU, two wavefronts per SIMD: pass 2 for head_dim 128 needs the registers (64
@@ -61,10 +70,23 @@ constexpr int kPfMinStages = 3;
 // with 6; 100 x 16000 of 12/2/128 76, 75, 68)
 constexpr int kPfSegStages = 6;
 
-// Stages of row group i (of S tokens x G heads) over T keys; at least one, so that a row group
+// Most stages of a row group of a short call that has n row groups of 128 rows: few leave ranges with
+// few parts to merge, many leave them with more starts.  Short against ranges, us: 12/2/128 16 x 300
+// (n = 2, 5 stages) 21.6, 25.8 and x 420 26.3, 25.4; 80 x 510 (8, 8) 29.8, 31.6 and x 540 31.8, 31.2; two
+// of 300 x 600 (60, 10) 34.2, 37.9 and x 768 38.4, 39.1.  14/2/64 16 x 540 (2, 9) 21.4, 21.6 and x 600
+// 22.8, 21.3; 80 x 660 (10, 11) 24.8, 25.6 and x 720 26.2, 25.3; 300 x 768 (34, 12) 26.5, 26.6 and x 900
+// 29.3, 27.1.
+__host__ __device__ constexpr int pf_short_stages(int D, int64_t n) {
+  return D == 128 ? (n < 4 ? 6 : n < 32 ? 8 : 10) : (n < 4 ? 9 : n < 32 ? 11 : 12);
+}
+// Workgroups that dequantize V beside pass 1's in a short call, at most.  By the row groups' own
+// workgroups after their stages: 11 x 300 of 12/2/128 27.6 -> 21.7 us, 80 x 80 17.3 -> 16.1.
+constexpr int kPfShortVWorkgroups = 512;
+
+// Stages of row group i of `rows` rows (of S tokens x G heads) over T keys; at least one, so that a row group
 // that sees nothing still has a workgroup to write its zeros.
-__host__ __device__ inline int pf_stages(int i, int S, int G, int T) {
-  const int last = min(S - 1, (kPfRows * (i + 1) - 1) / G);
+__host__ __device__ inline int pf_stages(int i, int rows, int S, int G, int T) {
+  const int last = min(S - 1, (rows * (i + 1) - 1) / G);
   return max(1, (T - S + last + kPfStage) / kPfStage);
 }
 
@@ -117,24 +139,30 @@ __device__ __forceinline__ float4* pf_slot(const AttnArgs& a, int D, int w0, int
                          : reinterpret_cast<float4*>(sync_parts(a)) + (id - a.pf_slots) * n;
 }
 
-template <int D, bool OUT>
-__global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(2)))
+// W wavefronts per workgroup: kPfWaves, or kPfShortWaves for short calls, which hold two LDS buffers
+// instead of three (a second barrier per stage) so that two workgroups fit a CU: 64 sequences of
+// 300 x 300 (12/2/128) 133 -> 93 us, one sequence the same either way.
+template <int D, bool OUT, int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_kernel(AttnArgs a, int layers) {
-  constexpr int W = kPfWaves, NTHR = 64 * W;
+  constexpr bool SHORT = W == kPfShortWaves;
+  constexpr int NTHR = 64 * W, ROWS = 32 * W;
+  constexpr int NB = SHORT ? 2 : 3, IDS = SHORT ? kPfShortIds : kPfIds;
+  static_assert(IDS % NTHR == 0 && IDS % 4 == 0, "the threads share the page ids evenly, whole stages of them");
   constexpr int KS = D / 16;        // MFMA steps of one q.k^T product over the head dimension
   constexpr int DT = D / 32;        // 32-dimension output tiles
   constexpr int CU = D / 16;        // 1 KiB chunks of one unit's K (and of its V)
   constexpr int PU = CU / 2;        // chunks per page block
   constexpr int NK = 2 * CU, NC = OUT ? 2 * NK : NK, CPW = NC / W;
   static_assert(CPW * W == NC && NK % W == 0, "the wavefronts share the chunks evenly");
-  __shared__ uint4 ring[3][NC * 64];
-  __shared__ int lpb[kPfIds];
+  __shared__ uint4 ring[NB][NC * 64];
+  __shared__ int lpb[IDS];
   __shared__ int s_scan[W], s_rest[W], s_pos[2], s_bad;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 5, n = lane & 31;
   const int nrg = a.pf_nrg, nf = a.B * nrg, LK = layers * a.KV;
 
   // a row group's weight in the order: its stages and, before them, the cost of its start
-  auto weight_of = [&](int f) { return kPfSegStages + pf_stages(f % nrg, a.S, a.G, seq_len_of(a, f / nrg)); };
+  auto weight_of = [&](int f) { return kPfSegStages + pf_stages(f % nrg, ROWS, a.S, a.G, seq_len_of(a, f / nrg)); };
 
   int window = 0;  // page-id windows staged so far
   if (tid == 0) s_bad = 0;
@@ -142,14 +170,14 @@ void prefill_kernel(AttnArgs a, int layers) {
   PfPos pos;
   int u = 0, uend = 0;       // current stage and end of the range
   int per1 = 0, per2 = 0;    // stages per workgroup of the two passes (0: whole row groups)
-  if ((OUT ? a.pf_w2 : a.pf_w1) == 0) {  // a row group per workgroup, the longest (last) ones first
+  if (SHORT || (OUT ? a.pf_w2 : a.pf_w1) == 0) {  // a row group per workgroup, the longest (last) ones first
     const int i = (int)blockIdx.x;
     pos.lk = i % LK;
-    pos.f = nf - 1 - i / LK;
+    pos.f = max(nf - 1 - i / LK, 0);
     pos.wt = weight_of(pos.f);
     pos.start = 0;
     u = 0;
-    uend = pos.wt;
+    uend = !SHORT || i < nf * LK ? pos.wt : 0;  // the workgroups past them dequantize V
   } else {
     // weights of the row groups of one (layer, KV head): each wavefront scans up to 64 of them in
     // its lanes, more are scanned NTHR at a time by the workgroup; `lo` of this thread's row
@@ -252,7 +280,7 @@ void prefill_kernel(AttnArgs a, int layers) {
 
     // this lane's row (of a wavefront without rows, or past the last, row R - 1: loaded, never
     // stored)
-    const int r = rg * kPfRows + wave * 32 + n;
+    const int r = rg * ROWS + wave * 32 + n;
     const bool rv = r < a.R;
     const int rc = min(r, a.R - 1), si = rc / a.G, hl = rc - si * a.G;
     const int lim = rv ? min(T - 1, T - a.S + si) : -1;
@@ -270,14 +298,14 @@ void prefill_kernel(AttnArgs a, int layers) {
     }
     // page ids of a window of the segment's blocks, to LDS
     auto stage_ids = [&](int wlo) {
-      const int blk0 = 4 * wlo, nids = 4 * min(kPfIds / 4, shi - wlo);
-      int id[kPfIds / NTHR];
+      const int blk0 = 4 * wlo, nids = 4 * min(IDS / 4, shi - wlo);
+      int id[IDS / NTHR];
 #pragma unroll
-      for (int i = 0; i < kPfIds / NTHR; ++i) id[i] = i * NTHR + tid < nids ? btrow[max(0, min(blk0 + i * NTHR + tid, nbk - 1))] : -1;
+      for (int i = 0; i < IDS / NTHR; ++i) id[i] = i * NTHR + tid < nids ? btrow[max(0, min(blk0 + i * NTHR + tid, nbk - 1))] : -1;
       ++window;
       __syncthreads();  // the ids before these are no longer read
 #pragma unroll
-      for (int i = 0; i < kPfIds / NTHR; ++i) {
+      for (int i = 0; i < IDS / NTHR; ++i) {
         const int j = i * NTHR + tid;
         if (j < nids) {
           const bool in = blk0 + j < nbk, ok = in && id[i] >= 0 && id[i] < a.num_blocks;
@@ -309,7 +337,7 @@ void prefill_kernel(AttnArgs a, int layers) {
     int kmin = rv ? lim : INT_MAX;
 #pragma unroll
     for (int off = 16; off > 0; off >>= 1) kmin = min(kmin, __shfl_xor(kmin, off));
-    const bool active = rg * kPfRows + wave * 32 < a.R;  // the wavefront has rows
+    const bool active = rg * ROWS + wave * 32 < a.R;  // the wavefront has rows
     const uint64_t rows = __ballot(rv);                  // the lanes that stand for one
     const int ufull = __builtin_amdgcn_readfirstlane(kmin == INT_MAX ? 0 : (kmin + 1) >> 5);
 
@@ -319,8 +347,8 @@ void prefill_kernel(AttnArgs a, int layers) {
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) acc[dt] = (f32x16)0.0f;
     }
-    for (int wlo = slo; wlo < shi; wlo += kPfIds / 4) {  // page-id windows; workgroup-uniform
-      const int nit = min(kPfIds / 4, shi - wlo);        // stages in the window
+    for (int wlo = slo; wlo < shi; wlo += IDS / 4) {  // page-id windows; workgroup-uniform
+      const int nit = min(IDS / 4, shi - wlo);           // stages in the window
       if (wlo > slo) stage_ids(wlo);
       const bool bad = __builtin_amdgcn_readfirstlane(s_bad) == window;  // an invalid id in the window
       // units of the window (32 keys): x = 0 .. 2 nit - 1, the first at key 32 * ux0
@@ -367,13 +395,21 @@ void prefill_kernel(AttnArgs a, int layers) {
       // score about as many of the VALU.  The first steps also write a chunk each of the next
       // stage, whose loads went out an iteration ago, to the third buffer, and send the loads of
       // the stage after it; the iteration's one barrier, at the end of the first unit, publishes
-      // the stage, so that the operand reads run on across iterations.
+      // the stage, so that the operand reads run on across iterations.  With two buffers the next
+      // stage's is the last one's: a barrier at the start, when every wavefront's products of it
+      // have gone out.
       constexpr int NM = OUT ? KS + 2 * DT : KS, SPM = 16 / NM, kAhead = OUT ? 4 : 2;
       constexpr int MS = (CPW + 1) & ~1;  // the steps that write and load chunks
       static_assert(CPW <= NM / 2, "kLater operand reads lie between the chunk writes and the barrier");
       constexpr int kLater = NM - MS < NM / 2 ? NM - MS : NM / 2;
       static_assert(KS == 2 * DT && NM * SPM == 16, "q.k^T and p.V steps alternate");
-      uint4 *cur = ring[0], *nxt = ring[1], *third = ring[2];
+      uint4 *cur = ring[0], *nxt = ring[1], *third = ring[NB - 1];
+      auto rotate = [&]() {
+        uint4* const t = cur;
+        cur = nxt;
+        nxt = NB == 2 ? t : third;
+        third = t;
+      };
       auto operand = [&](const uint4* sb, int m) {  // step m: of unit m / NM, k step or tile i
         const int un = m / NM, i = OUT ? (m % NM) / 2 : m % NM;
         const char* kb = reinterpret_cast<const char*>(sb) + kofs;
@@ -408,6 +444,13 @@ void prefill_kernel(AttnArgs a, int layers) {
         }
       };
       auto body = [&](int it, bool mask) {
+        if constexpr (NB == 2) {
+          __builtin_amdgcn_sched_barrier(0);
+          asm volatile("" ::: "memory");
+          __builtin_amdgcn_s_barrier();
+          asm volatile("" ::: "memory");
+          __builtin_amdgcn_sched_barrier(0);
+        }
         next_ids(it + 2);
         f32x16 sn = (f32x16)0.0f;
         uint32_t pn[8];
@@ -490,10 +533,7 @@ void prefill_kernel(AttnArgs a, int layers) {
             sc = sn;
           }
         }
-        uint4* const t = cur;
-        cur = nxt;
-        nxt = third;
-        third = t;
+        rotate();
       };
 
       // stage 0 and unit 0's K (slot 1 of stage -1), loaded together
@@ -531,6 +571,7 @@ void prefill_kernel(AttnArgs a, int layers) {
         for (; it < nit; ++it) body(it, true);
       } else {  // a wavefront without rows loads its share
         for (; it < nit; ++it) {
+          if constexpr (NB == 2) publish();
           next_ids(it + 2);
 #pragma unroll
           for (int j = 0; j < CPW; ++j) {
@@ -538,10 +579,7 @@ void prefill_kernel(AttnArgs a, int layers) {
             stg[j] = fetch1(it + 2, j);
           }
           publish();
-          uint4* const t = cur;
-          cur = nxt;
-          nxt = third;
-          third = t;
+          rotate();
         }
       }
       if constexpr (OUT) {  // the last unit's p.V
@@ -579,6 +617,7 @@ void prefill_kernel(AttnArgs a, int layers) {
     }
 
     // the next row group of the range
+    if constexpr (SHORT) break;
     u = next;
     if (u < uend) {
       pos.start = next;
@@ -599,7 +638,9 @@ void prefill_kernel(AttnArgs a, int layers) {
     typedef float f32x2 __attribute__((ext_vector_type(2)));
     const int nbmax = 2 * a.vh_stages;
     const int64_t items = (int64_t)LK * a.B * nbmax;
-    for (int64_t i = (int64_t)blockIdx.x * W + wave; i < items; i += (int64_t)gridDim.x * W) {
+    const int first = SHORT ? nf * LK : 0, wg = (int)blockIdx.x - first, wgs = (int)gridDim.x - first;
+    if (wg < 0) return;
+    for (int64_t i = (int64_t)wg * W + wave; i < items; i += (int64_t)wgs * W) {
       const int z = (int)(i / nbmax), blk = (int)(i - (int64_t)z * nbmax);
       const int zb = z / a.KV, kvh = z - zb * a.KV, layer = zb / a.B, b = zb - layer * a.B;
       const int T = seq_len_of(a, b), nbk = (T + kBlock - 1) / kBlock;

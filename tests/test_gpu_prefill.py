@@ -346,3 +346,74 @@ def test_prefill_empty_sequence(cuda_device, h, d, s, lens):
         elif i < 3 or i == b - 1:
             want = oatt.eager_attention(q[i:i + 1].cpu(), kc.cpu()[None][:, :, :n], v_hat[:, :, :n])
             assert_close(out[i:i + 1].cpu(), want, f"sequence {i} of {n}")
+
+
+@pytest.mark.parametrize("h,d,s,t", [(12, 128, 11, 11), (12, 128, 11, 384), (12, 128, 11, 385), (12, 128, 21, 64), (12, 128, 22, 65),
+                                     (12, 128, 64, 512), (12, 128, 64, 513), (12, 128, 400, 640), (14, 64, 10, 16), (14, 64, 19, 576),
+                                     (14, 64, 37, 577), (14, 64, 73, 704), (14, 64, 73, 705), (14, 64, 350, 768)])
+def test_prefill_short_contexts(cuda_device, h, d, s, t):
+    """Calls over few stages of keys take row groups of 128 rows, a workgroup of four wavefronts each:
+    one row group and the first rows of a second, one stage and one key past it, and both sides of
+    the rule's limits (6, 8, 10 and 9, 11, 12 stages by the number of row groups)."""
+    announce(f"prefill short {h}/2/{d} S={s} T={t}")
+    _prefill_case(cuda_device, h, 2, d, s, t, seed=810 + s + t, chunk_rows=128)
+
+
+@pytest.mark.parametrize("h,d", [(12, 128), (14, 64)])
+def test_prefill_short_ragged_batch_replays(cuda_device, h, d):
+    """Two layers of five short sequences (one shorter than the new rows, one empty) with invalid block
+    ids in one of them, recorded and replayed between eager calls: equal to the eager call, and
+    within the bar of the eager reference over the valid keys."""
+    announce(f"prefill short ragged batch {h}/2/{d}")
+    g = wl.gen(830 + d, cuda_device)
+    L, lens, s, kv = 2, [400, 45, 20, 0, 333], 45, 2
+    t, rows = max(lens), [0, 1, 2, 4]
+    cache = PagedKVCache(kv, d, num_layers=L, batch=5, num_blocks=sum(-(-x // 16) for x in lens) + 5, device=cuda_device,
+                         seed=831, growable=False)
+    slots = None
+    for layer in range(L):
+        k = torch.randn((sum(lens), kv, d), generator=g, device=cuda_device).to(torch.bfloat16)
+        v = torch.randn((sum(lens), kv, d), generator=g, device=cuda_device).to(torch.bfloat16)
+        slots = cache.prefill(layer, k, v, lens, slots)
+    table = cache.block_table().clone()
+    holes = [0, 7, 20]
+    table[4, holes] = torch.tensor([-1, 1 << 20, cache.alloc.num_blocks], dtype=torch.int32, device=cuda_device)
+    sl = cache.seq_lens_tensor()
+    q = torch.randn((L, 5, s, h, d), generator=g, device=cuda_device).to(torch.bfloat16)
+    ws = ops.new_workspace(cuda_device, ops.attention_workspace_bytes(L, 5, h, kv, s, d, t))
+
+    def call(out=None):
+        return ops.paged_attention(q, cache.k_pages, cache.v_pages, cache.v_scales, table, sl, t, q_token_major=True, out=out,
+                                   workspace_tensor=ws)
+
+    want = call()
+    out = torch.empty_like(q)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), "a replay differs from the eager call"
+        assert torch.equal(call(), want)
+    torch.cuda.synchronize()
+    for layer in range(L):
+        assert not want[layer, 3].any()
+        for b in rows:
+            n = lens[b]
+            kc, vc, sc = cache.gather(layer, b)
+            v_hat = oq.dequantize_kv_fp8(vc.cpu()[None], sc.cpu()[None], torch.bfloat16)
+            keep = torch.ones(n, dtype=torch.bool)
+            for j in holes if b == 4 else []:
+                keep[16 * j:16 * j + 16] = False
+            pos = torch.nonzero(keep).flatten()
+            for i in (0, 1, 26, s - 1):
+                m = int((pos <= n - s + i).sum())
+                got = want[layer, b, i].cpu()[None, :, None]
+                if m == 0:
+                    assert not got.any(), f"row {i} of sequence {b} sees no key"
+                    continue
+                ref = oatt.eager_attention(q[layer, b, i].cpu()[None, :, None], kc.cpu()[None][:, :, pos[:m]], v_hat[:, :, pos[:m]])
+                assert_close(got, ref, f"layer {layer} sequence {b} row {i}")

@@ -4,7 +4,8 @@ A prefill call's row groups (256 rows) hold stages of 64 keys; each launch gives
 contiguous range of the stages of all row groups, weighted by what starting one costs.  Whatever the
 shapes and the actual lengths (the plan is made for the longest sequence), every stage of every
 row group must belong to exactly one workgroup, the segments of a row group must fit its statistics,
-and every part slot must be its segment's own and lie inside the workspace.
+and every part slot must be its segment's own and lie inside the workspace.  Calls over short
+contexts take whole row groups of 128 rows instead.
 """
 import random
 
@@ -12,7 +13,7 @@ import pytest
 
 from specdec_amd import _native
 
-ROWS, STAGE, SEG, MIN, CUS = 256, 64, 6, 3, 256
+ROWS, SHORT_ROWS, STAGE, SEG, MIN, CUS = 256, 128, 64, 6, 3, 256
 SYNC_PART, DESC, MAX_GROUPS = 8 << 20, (1 << 14) * 8, 1 << 14
 
 
@@ -20,9 +21,17 @@ def cdiv(a, b):
     return -(-a // b)
 
 
-def stages(i, s, g, t):
-    last = min(s - 1, (ROWS * (i + 1) - 1) // g)
+def stages(i, s, g, t, rows=ROWS):
+    last = min(s - 1, (rows * (i + 1) - 1) // g)
     return max(1, (t - s + last + STAGE) // STAGE if t - s + last + STAGE > 0 else 0)
+
+
+def short(groups, r, s, g, d, t):
+    """Whether the call takes whole row groups of 128 rows."""
+    nrg = cdiv(r, SHORT_ROWS)
+    n = groups * nrg
+    most = (6 if n < 4 else 8 if n < 32 else 10) if d == 128 else (9 if n < 4 else 11 if n < 32 else 12)
+    return stages(nrg - 1, s, g, t, SHORT_ROWS) <= most
 
 
 def plan(groups, r, s, g, d, t):
@@ -49,6 +58,8 @@ def plan(groups, r, s, g, d, t):
     have = slots + (SYNC_PART - DESC) // slot_b
     n = groups * nrg
     w2 = min(CUS, max(have // 2, have - n), cdiv(u, MIN))
+    if short(groups, r, s, g, d, t):
+        return total, 0, 0, MIN, split, slots, False, have
     if u >= 1 << 30 or nbk >= 1 << 22 or n > MAX_GROUPS or w2 < min(n, CUS):
         return total, 0, 0, MIN, split, slots, False, have
     w1, min1 = 0, MIN
@@ -108,7 +119,7 @@ def test_ranges_cover_every_stage_once(seed):
     rng = random.Random(seed)
     lib = _native.load()
     split = 0
-    for _ in range(40):
+    for _ in range(60):
         d, g = rng.choice([(128, 6), (64, 7)])
         kv, layers, b = rng.choice([1, 2]), rng.choice([1, 1, 2, 5]), rng.choice([1, 1, 2, 3, 9])
         s = int(2 ** rng.uniform(3.6, 11))
