@@ -218,3 +218,28 @@ def test_varlen_prefill_tile_table(cuda_device, d):
     assert np.array_equal(bits16(kp[0]), ek)
     assert torch.equal(vp, vp2) and torch.equal(vs.view(torch.int32), vs2.view(torch.int32))
     assert torch.equal(kp.view(torch.int16), kp2.view(torch.int16))
+
+
+@pytest.mark.parametrize("d", [128, 64])
+@pytest.mark.parametrize("n", [63 * 16, 64 * 16 - 1, 64 * 16 + 1, 129 * 16 + 5])
+@pytest.mark.parametrize("start", [0, 5])
+def test_rows_around_runs_of_tiles(cuda_device, d, n, start):
+    """Tiles are dealt to the XCDs in runs of 64: one tile less than a run, a run, one more and two runs,
+    rows that start a page block and rows that share every block between two tiles."""
+    announce(f"quant runs of tiles d={d} n={n} start={start}")
+    g = wl.gen(41 + n)
+    kv, nb = 2, (n + start) // 16 + 3
+    v, k = wl.randn_bf16((n, kv, d), g), wl.randn_bf16((n, kv, d), g)
+    blocks = torch.randperm(nb, generator=g).numpy()
+    slots = np.asarray(opaged.slots_for(blocks, start, n), dtype=np.int32)
+    kp, vp, vs = _pages(cuda_device, 1, nb, kv, d)
+    ops.quant_append(v.to(cuda_device), to_dev(slots, cuda_device), kp[0], vp[0], vs[0], k.to(cuda_device))
+    torch.cuda.synchronize()
+    q, s = quantize_rows(v)
+    ek, ev, es = opaged.alloc(nb, kv, d)
+    opaged.write(ek, ev, es, bits16(k), q, s, slots)
+    blk, off = slots // 16, slots % 16
+    assert np.array_equal(vp[0].cpu().numpy()[blk, :, :, off], ev[blk, :, :, off])
+    assert np.array_equal(vs[0].cpu().numpy()[blk, :, off], es[blk, :, off])
+    assert np.array_equal(bits16(kp[0])[blk, :, :, off, :], ek[blk, :, :, off, :])
+    assert int((vp[0].cpu() != 0xA5).any(2).sum()) <= kv * n     # nothing past the rows
