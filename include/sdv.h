@@ -126,8 +126,8 @@ size_t sdv_attention_workspace_size(int32_t num_layers, int32_t batch, int32_t q
  * Zero the workspace's synchronisation area (its first SDV_SYNC_BYTES bytes) on `stream`.
  * Call it once after allocating a workspace and before its first sdv_paged_attention; every
  * call that completes normally leaves the statistics zero again (the partial slots keep the
- * last call's values; each item zeroes its own slot at the start of the next call).  No
- * counterpart in the reference (it has no workspace).
+ * last call's values, those of prefill rows among them; each item zeroes its own slot at the start
+ * of the next single launch).  No counterpart in the reference (it has no workspace).
  *
  * The single-launch path exchanges (max, sum) statistics between workgroups through this
  * area as 64-bit (value, call tag) words; a reader takes a word only when it carries its own
@@ -176,7 +176,7 @@ int sdv_attention_set_wait_limit(uint32_t polls);
  * Which path sdv_paged_attention takes for these sizes on the current device: the number of
  * workgroups of the single-launch kernel, or 0 when another path serves the call (several
  * query-row groups, or a problem the device cannot hold at once: the persistent per-group
- * kernel for 256 or more one-tile groups, else three launches).  A batch of 2..64 sequences
+ * kernel for 256 or more one-tile groups, the prefill kernels, else three launches).  A batch of 2..64 sequences
  * is taken to pass per-sequence lengths: its single launch uses every workgroup the device
  * holds and sizes each sequence's items from its length.  Queries the device's occupancy; no
  * launch.  No counterpart in the reference.

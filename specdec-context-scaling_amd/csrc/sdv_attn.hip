@@ -2131,7 +2131,8 @@ static bool make_plan(int L, int B, int H, int KV, int S, int D, int max_seq_len
     plan_prefill(groups, (int)R, S, G, D, max_seq_len, p);
     return true;
   }
-  // the sync area [0, kSyncBytes) is shared by every layout and only the fused kernel uses it
+  // the sync area [0, kSyncBytes) is shared by every layout; the fused kernel uses it, the group
+  // kernel its words 2-3 and the prefill its partials
   const size_t scores = round_up((size_t)(groups * R * p->score_stride * 2), 256);
   const size_t stats = round_up((size_t)(groups * p->n_qk_chunks * p->rpad * 8), 256);
   const size_t partial = round_up((size_t)(groups * p->n_pv_chunks * R * D * 4), 256);

@@ -221,6 +221,19 @@ def test_prefill_many_row_groups_and_windows(cuda_device):
         assert_close(out[i:i + 1].transpose(1, 2).cpu(), want, f"sequence {i}")
 
 
+@pytest.mark.parametrize("h,d,s,t", [(12, 128, 2048, 131072), (14, 64, 1500, 150001)])
+def test_prefill_ranges_over_page_id_windows(cuda_device, h, d, s, t):
+    """Ranges of more than 512 stages stage their page ids in several windows of 2,048 that begin where
+    the range does (769 stages a workgroup for 2048 rows over 128K keys, 768 and more for 1500 over
+    150,001); the first, two middle and the last rows are checked."""
+    announce(f"prefill {h}/2/{d} S={s} T={t} page-id windows inside ranges")
+    rows = 256
+    stages = sum(6 + (t - s + min(s - 1, (rows * (i + 1) - 1) // (h // 2)) + 64) // 64 for i in range(-(-s * (h // 2) // rows)))
+    assert 2 * stages > 256 * 512, "a workgroup's range is longer than a window"
+    _prefill_case(cuda_device, h, 2, d, s, t, seed=755 + d,
+                  check_rows=[(0, 4), (s // 3, s // 3 + 4), (s // 2, s // 2 + 4), (s - 4, s)])
+
+
 @pytest.mark.parametrize("h,d,s,t", [(12, 128, 300, 1500), (14, 64, 96, 900)])
 def test_prefill_late_maximum(cuda_device, h, d, s, t):
     """Pass 1 takes its exponentials against an earlier maximum and goes through the online update

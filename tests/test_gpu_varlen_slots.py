@@ -36,27 +36,38 @@ def test_varlen_slots_match_the_host(cuda_device, lengths):
 
 
 def test_prefill_tables_follow_lengths_and_streams(cuda_device):
-    """prefill reuses a table only for the same lengths on the same stream."""
+    """One pool, several lengths and streams in turn: prefill builds its table again when the lengths or
+    the stream change, takes the same one when neither does, and writes the pages of every call
+    where they belong."""
     announce("prefill tables per lengths and stream")
     g = torch.Generator(device="cuda")
     g.manual_seed(4)
-    k = torch.randn((50, 2, 64), generator=g, device="cuda").to(torch.bfloat16)
     side = torch.cuda.Stream()
-    for lengths in ([20, 30], [30, 20], [30, 20]):
-        for stream in (torch.cuda.current_stream(), side):
-            cache = PagedKVCache(2, 64, batch=2, num_blocks=6, device=cuda_device, seed=5)
-            ref = PagedKVCache(2, 64, batch=2, num_blocks=6, device=cuda_device, seed=5)
-            with torch.cuda.stream(stream):
-                stream.wait_stream(torch.cuda.default_stream())
-                for _ in range(2):
-                    cache.prefill(0, k, k, lengths)
-            torch.cuda.synchronize()
-            for b in range(2):
-                ref.reserve(b, lengths[b])
-            ops.quant_append(k, _host(ref, lengths)[0].cuda(), *ref.layer(0), k)
-            torch.cuda.synchronize()
-            assert torch.equal(cache.k_pages, ref.k_pages) and torch.equal(cache.v_pages, ref.v_pages)
-    assert cache._tiles[:2] == ((30, 20), side.cuda_stream)
+    cache, ref = (PagedKVCache(2, 64, batch=2, num_blocks=6, device=cuda_device, seed=5) for _ in range(2))
+    for b in range(2):
+        cache.reserve(b, 40)
+        ref.reserve(b, 40)
+    last = None
+    for lengths, stream in (([20, 30], None), ([30, 20], None), ([30, 20], None), ([30, 20], side), ([30, 20], side),
+                            ([20, 30], side), ([20, 30], None), ([17, 33], None), ([17, 33], side)):
+        k = torch.randn((50, 2, 64), generator=g, device="cuda").to(torch.bfloat16)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream or torch.cuda.current_stream()):
+            slots = cache.prefill(0, k, k, lengths)
+            table = cache._tiles[2]
+            cache.prefill(0, k, k, lengths, slots)
+            assert cache._tiles[2] is table, "same lengths, same stream, slots passed: same table"
+        torch.cuda.synchronize()
+        key = (tuple(lengths), (stream or torch.cuda.current_stream()).cuda_stream)
+        assert cache._tiles[:2] == key
+        assert torch.equal(cache._tiles[2].cpu(), _host(cache, lengths)[1])
+        if last is not None and last[0] != key:
+            assert cache._tiles[2] is not last[1], "other lengths or another stream: another table"
+        last = key, cache._tiles[2]
+        ops.quant_append(k, _host(ref, lengths)[0].cuda(), *ref.layer(0), k)
+        torch.cuda.synchronize()
+        for x, y in zip(cache.layer(0), ref.layer(0)):
+            assert torch.equal(x, y)
 
 
 def test_varlen_slots_refuse_unreserved_positions(cuda_device):
